@@ -402,6 +402,61 @@ __device__ __forceinline__ float inv_of(float scale) {
   return (float)(1.0 / (double)scale);
 }
 
+// ---- which grads the norm passes leave in the memory-side cache --------------
+// Every grad is read twice in a step: by the norm pass, then by the update.
+// A load with the nontemporal hint passes the 256 MB memory-side cache by, a
+// plain one leaves its line there, and the update's own streams (all
+// nontemporal) do not evict it. So the norm passes read the first
+// kKeepBytes of the grads, in the order in which the update takes them, with
+// plain loads and the rest, which would only evict those, nontemporally; the
+// update's grad loads then find them in the cache: 2 of the step's 30 bytes an
+// element (4 of 32 with fp32 grads) do not come from HBM again. Flat steps on
+// MI355X, one process, with 0 / 128 / 192 / 256 / 320 MB kept and with every
+// load plain, us: 1.24e8 bf16 elements (248 MB of grads) 616 / 599 / 591 /
+// 584 / 584 / 584; 6.0e7 fp32 (240 MB) 320 / 307 / 298 / 293 / 293 / 293;
+// 2.5e8 bf16 (500 MB) 1246 / 1228 / 1219 / 1209 / 1209 / 1210; 1.0e9 bf16
+// 4981 / 4958 / 4951 / 4940 / 4940 / 4971. Below 3e6 elements both are the same.
+constexpr int64_t kKeepBytes = int64_t(1) << 28;
+
+// Trips of U 16-byte slots per thread over slots [i0, end) of nvec, each
+// slot's term added by add(slot, acc) in slot order; leaves i0 at the next
+// trip's slot.
+template <int U, bool NT, class Add>
+__device__ __forceinline__ double norm_trips(const u4* g16, int64_t nvec, int64_t end, int64_t stride, int64_t lanes,
+                                             int64_t lane, int64_t& i0, double acc, Add add) {
+  for (; i0 - lane < end; i0 += stride) {
+    u4 S[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = i0 + u * lanes;
+      S[u] = (i < nvec) ? ld<NT>(g16 + i) : u4{0u, 0u, 0u, 0u};  // zeros add nothing to any norm
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc = add(S[u], acc);
+  }
+  return acc;
+}
+
+// A flat norm pass: the trips that start below slot `keep` with plain loads,
+// the others nontemporally. (Two loops: in one, the compiler merges the two
+// kinds of load and drops the hint.)
+template <int U, class Add>
+__device__ __forceinline__ double norm_sweep(const u4* g16, int64_t nvec, int64_t keep, Add add) {
+  const int64_t stride = (int64_t)gridDim.x * kBlock * U;
+  int64_t i0 = (int64_t)blockIdx.x * kBlock * U + threadIdx.x;
+  double acc = norm_trips<U, false>(g16, nvec, keep < nvec ? keep : nvec, stride, kBlock, threadIdx.x, i0, 0.0, add);
+  return norm_trips<U, true>(g16, nvec, nvec, stride, kBlock, threadIdx.x, i0, acc, add);
+}
+
+// One chunk of a ragged norm pass by `lanes` threads (this one is `lane`).
+template <int U, class Add>
+__device__ __forceinline__ double norm_chunk(const u4* g16, int64_t nvec, bool keep, int64_t lanes, int64_t lane,
+                                             double acc, Add add) {
+  int64_t i0 = lane;
+  if (keep) return norm_trips<U, false>(g16, nvec, nvec, lanes * U, lanes, lane, i0, acc, add);
+  return norm_trips<U, true>(g16, nvec, nvec, lanes * U, lanes, lane, i0, acc, add);
+}
+
 // ---- K1: unscale + inf/NaN + squared norm ----------------------------------
 // Each element contributes (double)(f32(g) * inv)^2. The square of a finite
 // fp32 value is exact in fp64 and the sum of 2^31 of them cannot overflow,
@@ -413,10 +468,10 @@ __device__ __forceinline__ float inv_of(float scale) {
 // blocks read those two fields, which nothing else writes during the step,
 // while one of them writes the state's updated fields.
 
-template <int GD, int U, bool NT>
+template <int GD, int U>
 __global__ __launch_bounds__(kBlock) void k1_unscale_norm(const void* __restrict__ gv, int64_t n,
                                                           const DsxState* state, double* __restrict__ partials,
-                                                          DsxState* fold) {
+                                                          DsxState* fold, int64_t keep) {
   using G = Grad<GD>;
   const float inv = inv_of(state->scale);
   if (fold != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -428,18 +483,7 @@ __global__ __launch_bounds__(kBlock) void k1_unscale_norm(const void* __restrict
   const u4* g16 = static_cast<const u4*>(gv);
   const typename G::elem* g = static_cast<const typename G::elem*>(gv);
   const int64_t nvec = n / G::per16;
-  const int64_t stride = (int64_t)gridDim.x * kBlock * U;
-  double acc = 0.0;
-  for (int64_t i0 = (int64_t)blockIdx.x * kBlock * U + threadIdx.x; i0 < nvec; i0 += stride) {
-    u4 S[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t i = i0 + (int64_t)u * kBlock;
-      S[u] = (i < nvec) ? ld<NT>(g16 + i) : u4{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) acc = G::sumsq16(S[u], inv, acc);
-  }
+  double acc = norm_sweep<U>(g16, nvec, keep, [inv](const u4& v, double x) { return G::sumsq16(v, inv, x); });
   const int64_t tail0 = nvec * G::per16;
   const int64_t gt = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (gt < n - tail0) {
@@ -457,25 +501,15 @@ __global__ __launch_bounds__(kBlock) void k1_unscale_norm(const void* __restrict
 template <int GD, int K>
 __global__ __launch_bounds__(kBlock) void k1_norm(const void* __restrict__ gv, int64_t n,
                                                   const DsxState* __restrict__ state, double p,
-                                                  double* __restrict__ partials) {
+                                                  double* __restrict__ partials, int64_t keep) {
   using G = Grad<GD>;
   constexpr int U = 4;
   const float inv = inv_of(state->scale);
   const u4* g16 = static_cast<const u4*>(gv);
   const typename G::elem* g = static_cast<const typename G::elem*>(gv);
   const int64_t nvec = n / G::per16;
-  const int64_t stride = (int64_t)gridDim.x * kBlock * U;
-  double acc = 0.0;
-  for (int64_t i0 = (int64_t)blockIdx.x * kBlock * U + threadIdx.x; i0 < nvec; i0 += stride) {
-    u4 S[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t i = i0 + (int64_t)u * kBlock;
-      S[u] = (i < nvec) ? ld<true>(g16 + i) : u4{0u, 0u, 0u, 0u};  // zeros add nothing to any kind
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) acc = norm_acc16<GD, K>(S[u], inv, p, acc);
-  }
+  double acc = norm_sweep<U>(g16, nvec, keep,
+                             [inv, p](const u4& v, double x) { return norm_acc16<GD, K>(v, inv, p, x); });
   const int64_t tail0 = nvec * G::per16;
   const int64_t gt = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (gt < n - tail0) acc = norm_acc<K>(acc, G::one(g[tail0 + gt]) * inv, p);
@@ -487,11 +521,12 @@ template <int GD, int K>
 __global__ __launch_bounds__(kBlock) void k1_norm_multi(const DsxTensorRef* __restrict__ tensors,
                                                         const DsxChunk* __restrict__ chunks, int64_t nchunks,
                                                         const DsxState* __restrict__ state, double p,
-                                                        double* __restrict__ partials) {
+                                                        double* __restrict__ partials, int64_t keep) {
   using G = Grad<GD>;
   constexpr int U = 4;
   const float inv = inv_of(state->scale);
   double acc = 0.0;
+  int64_t seen = 0;  // elements this block has read
   for (int64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
     const DsxChunk ch = chunks[c];
     const typename G::elem* g = static_cast<const typename G::elem*>(tensors[ch.tensor].grad) + ch.start;
@@ -500,19 +535,12 @@ __global__ __launch_bounds__(kBlock) void k1_norm_multi(const DsxTensorRef* __re
     if (aligned16(g)) {
       const u4* g16 = reinterpret_cast<const u4*>(g);
       const int64_t nvec = len / G::per16;
-      for (int64_t i0 = threadIdx.x; i0 < nvec; i0 += kBlock * U) {
-        u4 S[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int64_t i = i0 + (int64_t)u * kBlock;
-          S[u] = (i < nvec) ? ld<true>(g16 + i) : u4{0u, 0u, 0u, 0u};
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) acc = norm_acc16<GD, K>(S[u], inv, p, acc);
-      }
+      acc = norm_chunk<U>(g16, nvec, seen < keep, kBlock, threadIdx.x, acc,
+                          [inv, p](const u4& v, double x) { return norm_acc16<GD, K>(v, inv, p, x); });
       done = nvec * G::per16;
     }
     for (int64_t e = done + threadIdx.x; e < len; e += kBlock) acc = norm_acc<K>(acc, G::one(g[e]) * inv, p);
+    seen += len;
   }
   const double s = block_reduce<K>(acc);
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
@@ -1168,7 +1196,8 @@ template <int GD, bool WAVE>
 __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorRef* __restrict__ tensors,
                                                                 const DsxChunk* __restrict__ chunks,
                                                                 int64_t nchunks, const DsxState* state,
-                                                                double* __restrict__ partials, DsxState* fold) {
+                                                                double* __restrict__ partials, DsxState* fold,
+                                                                int64_t keep) {
   using G = Grad<GD>;
   constexpr int U = 4;
   constexpr int kWaves = kBlock / 64;
@@ -1181,6 +1210,7 @@ __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorR
     fold->clip_once = 0;
   }
   double acc = 0.0;
+  int64_t seen = 0;  // elements this block (or wave) has read
   const int lane = WAVE ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
   const int64_t stride = WAVE ? (int64_t)gridDim.x * kWaves : (int64_t)gridDim.x;
   int64_t c = WAVE ? (int64_t)blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)
@@ -1195,22 +1225,15 @@ __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorR
       if (aligned16(g)) {
         const u4* g16 = reinterpret_cast<const u4*>(g);
         const int64_t nvec = ch.len / G::per16;
-        for (int64_t i0 = lane; i0 < nvec; i0 += kLanes * U) {
-          u4 S[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int64_t i = i0 + (int64_t)u * kLanes;
-            S[u] = (i < nvec) ? ld<true>(g16 + i) : u4{0u, 0u, 0u, 0u};
-          }
-#pragma unroll
-          for (int u = 0; u < U; ++u) acc = G::sumsq16(S[u], inv, acc);
-        }
+        acc = norm_chunk<U>(g16, nvec, seen < keep, kLanes, lane, acc,
+                            [inv](const u4& v, double x) { return G::sumsq16(v, inv, x); });
         done = nvec * G::per16;
       }
       for (int64_t e = done + lane; e < ch.len; e += kLanes) {
         const float a = G::one(g[e]) * inv;
         acc = __builtin_fma((double)a, (double)a, acc);
       }
+      seen += ch.len;
       if (cn >= nchunks) break;
       c = cn;
       ch = chn;
@@ -1456,13 +1479,19 @@ __global__ __launch_bounds__(kBlock) void k3_adamw_fold(const DsxTensorRef* __re
 
 hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
+// kKeepBytes as a bound for a norm pass: in 16-byte slots of a flat buffer,
+// or in elements for each of the walkers (blocks or waves) that share a list.
+// The nontemporal hint switched off: every load plain.
+int64_t keep_slots() { return g_tune.nontemporal ? kKeepBytes / 16 : INT64_MAX; }
+int64_t keep_elems(int gdt, int64_t walkers) {
+  return g_tune.nontemporal ? ceil_div(kKeepBytes / (gdt == DSX_F32 ? 4 : 2), walkers) : INT64_MAX;
+}
+
 template <int GD>
 void launch_k1(const void* g, int64_t n, const DsxState* st, double* partials, int nparts, DsxState* fold,
                hipStream_t s) {
-  if (g_tune.nontemporal)
-    hipLaunchKernelGGL((k1_unscale_norm<GD, 4, true>), dim3(nparts), dim3(kBlock), 0, s, g, n, st, partials, fold);
-  else
-    hipLaunchKernelGGL((k1_unscale_norm<GD, 4, false>), dim3(nparts), dim3(kBlock), 0, s, g, n, st, partials, fold);
+  hipLaunchKernelGGL((k1_unscale_norm<GD, 4>), dim3(nparts), dim3(kBlock), 0, s, g, n, st, partials, fold,
+                     keep_slots());
 }
 
 template <int GD, int PD, int U, bool NT, bool DRAIN>
@@ -1774,9 +1803,9 @@ void launch_norm_k(bool multi, const void* g, int64_t n, const DsxTensorRef* t, 
                    const DsxState* st, double p, double* partials, int nparts, hipStream_t s) {
   const dim3 grid((unsigned)nparts), blk(kBlock);
   if (multi)
-    hipLaunchKernelGGL((k1_norm_multi<GD, K>), grid, blk, 0, s, t, c, nc, st, p, partials);
+    hipLaunchKernelGGL((k1_norm_multi<GD, K>), grid, blk, 0, s, t, c, nc, st, p, partials, keep_elems(GD, nparts));
   else
-    hipLaunchKernelGGL((k1_norm<GD, K>), grid, blk, 0, s, g, n, st, p, partials);
+    hipLaunchKernelGGL((k1_norm<GD, K>), grid, blk, 0, s, g, n, st, p, partials, keep_slots());
 }
 
 template <int GD>
@@ -1878,10 +1907,10 @@ void launch_k1_multi(bool wave, dim3 grid, const DsxTensorRef* tensors, const Ds
                      const DsxState* state, double* partials, DsxState* fold, hipStream_t s) {
   if (wave)
     hipLaunchKernelGGL((k1_unscale_norm_multi<GD, true>), grid, dim3(kBlock), 0, s, tensors, chunks, nchunks,
-                       state, partials, fold);
+                       state, partials, fold, keep_elems(GD, (int64_t)grid.x * kWaves));
   else
     hipLaunchKernelGGL((k1_unscale_norm_multi<GD, false>), grid, dim3(kBlock), 0, s, tensors, chunks, nchunks,
-                       state, partials, fold);
+                       state, partials, fold, keep_elems(GD, grid.x));
 }
 
 // K1 over a chunk table. Each wave takes its own chunks when the table has
