@@ -716,8 +716,8 @@ def link_ceiling(dev) -> dict:
 
 def measure_offload(dev, full: int, budget_gib: float, steps: int) -> dict:
     """Llama-3-70B ZeRO-3 one-rank shard, 8,819,213,312 elements,
-    fp32 master/m/v in pinned host memory (105.8 GB) streamed through HBM in
-    64 Mi-element chunks, bf16 grads N(0, 3e-4^2) and params in HBM; AdamW lr
+    fp32 master/m/v in pinned host memory (105.8 GB), which K2 reads and
+    writes in place over the host link, bf16 grads N(0, 3e-4^2) and params in HBM; AdamW lr
     1.5e-4, betas (0.9, 0.95), wd 0.1. Bound by the host link (12 B/elt each
     way), so the figure of merit is link GB/s against the measured link
     ceiling, not HBM TB/s."""
@@ -775,16 +775,17 @@ def measure_offload(dev, full: int, budget_gib: float, steps: int) -> dict:
         times.append(time.perf_counter() - t0)
         _progress(f"step {i + 1}: {times[-1]:.3f} s")
     s = ops.read_state(st)
-    # The link measured right after the timed steps, in this process, on the
-    # step's own copy streams and pinned buffers; the ceiling is the larger
-    # of this and the fresh process's figure.
-    _progress("measuring the host link on the step's own streams")
+    # The link measured right after the timed steps, in this process, by plain
+    # copies on the streamer's copy streams and the step's pinned buffers; the
+    # ceiling is the larger of this and the fresh process's figure. The step's
+    # own kernel, which paces its requests to the link, can pass it.
+    _progress("measuring the host link with copies")
     from distributedspeed_amd.offload import measure_streamer_link
-    # the copy-only schedule is also started as a step starts it, behind K1
-    # (which reads the grads and writes the partials, and changes no state)
+    # the copy-only schedule is also started behind K1, as the step is
+    # (K1 reads the grads and writes the partials, and changes no state)
     link_here = measure_streamer_link(streamer, (master, m, v), pipeline_passes=3,
                                       lead=lambda: ops.unscale_norm(grad, st, parts, nparts))
-    link_here["measured_in"] = "this process, the step's copy streams and pinned buffers, after the timed steps"
+    link_here["measured_in"] = "this process, copies on the streamer's streams and the step's pinned buffers, after the timed steps"
     ceiling = max(link["both_each_way"], link_here["both_each_way"])
     sec = sorted(times)[len(times) // 2]
     each_way = 12 * n / sec / 1e9

@@ -231,6 +231,26 @@ def plan_adamw_flat(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: tor
                   gdt, ctypes.c_int64(n), _ptr(scalars), keep=(master, exp_avg, exp_avg_sq, param16, grad, scalars))
 
 
+def adamw_host_state(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: torch.Tensor,
+                     param16: torch.Tensor | None, grad: torch.Tensor, scalars: torch.Tensor) -> None:
+    """K2 with the fp32 state in pinned host memory, in place over the host
+    link; param16, grad and scalars on the GPU whose stream it runs on."""
+    dev = _device(grad)
+    n = grad.numel()
+    host = torch.device("cpu")
+    for name, t in (("master", master), ("exp_avg", exp_avg), ("exp_avg_sq", exp_avg_sq)):
+        _need(t, name, torch.float32, n, host)
+    _need(grad, "grad", None, n, dev)
+    gdt = grad_code(grad.dtype)
+    pdt = DSX_F16
+    if param16 is not None:
+        _need(param16, "param16", None, n, dev)
+        pdt = dtype_code(param16.dtype)
+    _need(scalars, "scalars", torch.uint8, SCALARS_BYTES, dev, 8)
+    _lib.call("dsx_adamw_host_state", _ptr(master), _ptr(exp_avg), _ptr(exp_avg_sq), _ptr(param16), pdt, _ptr(grad),
+              gdt, ctypes.c_int64(n), _ptr(scalars), _stream(dev))
+
+
 def traffic_probe_flat(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: torch.Tensor,
                        param16: torch.Tensor, grad: torch.Tensor) -> None:
     """Measurement only: K2's traffic in K2's launch shape without the AdamW

@@ -396,6 +396,17 @@ int dsx_adamw_flat(float* master, float* exp_avg, float* exp_avg_sq,
                    int grad_dtype, int64_t n, const DsxStepScalars* scalars,
                    void* stream);
 
+/* dsx_adamw_flat with master/exp_avg/exp_avg_sq in pinned HOST memory
+ * (hipHostMalloc), read and written in place over the host link; param16,
+ * grad and scalars are device memory. DSX_EINVAL for host memory that is not
+ * pinned. Replaces the copies to and from the GPU around the step at
+ * Src/zero/stage1.py:376-398, 482-498 and Src/zero/stage2.py:432-454,
+ * 563-582. */
+int dsx_adamw_host_state(float* master, float* exp_avg, float* exp_avg_sq,
+                         void* param16, int param_dtype, const void* grad,
+                         int grad_dtype, int64_t n,
+                         const DsxStepScalars* scalars, void* stream);
+
 /* Measurement only, no counterpart in the reference: K2's exact traffic
  * (grad, master, exp_avg and exp_avg_sq read; master, exp_avg, exp_avg_sq
  * and param16 written: 28 B per element) in K2's launch shape for n, with

@@ -1,0 +1,98 @@
+"""K2 on fp32 state in pinned host memory (dsx_adamw_host_state): the same bits
+as K2 on the same state in HBM, at the edges of its slots, trips and grid, and
+through the offloaded step; host memory that is not pinned is refused by the
+entry point and staged by the streamer."""
+from __future__ import annotations
+
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TRIP = 256 * 2 * 4  # elements of a block's trip
+
+
+def _say(msg):
+    print(f"[gpu-test] {msg}", file=sys.stderr, flush=True)
+
+
+def _inputs(n, gdt, pdt, gpu, seed):
+    import torch
+    gen = torch.Generator(device=gpu).manual_seed(seed)
+    p, m = (torch.empty(n, device=gpu).normal_(0.0, 0.02, generator=gen) for _ in range(2))
+    v = torch.empty(n, device=gpu).uniform_(0.0, 1e-6, generator=gen)
+    g = torch.empty(n, device=gpu).normal_(0.0, 1e-3, generator=gen).to(gdt)
+    return p, m, v, (p.to(pdt) if pdt is not None else None), g
+
+
+def _scalars(gpu, skip=0):
+    from distributedspeed_amd import ops
+    from distributedspeed_amd._lib import DsxStepScalars
+    sc = DsxStepScalars()
+    sc.inv_scale, sc.clip_coef, sc.decay, sc.w1, sc.w1c = 1.0, 0.5, 0.9999, 0.1, 0.9
+    sc.b2, sc.val2, sc.eps, sc.bc2s, sc.nss, sc.skip = 0.999, 0.001, 1e-8, 0.3, -1e-3, skip
+    return ops.scalars_from_host(sc, gpu)
+
+
+def _pinned(t):
+    import torch
+    from distributedspeed_amd.offload import pinned_empty
+    h = pinned_empty(t.numel())
+    h.copy_(t)
+    torch.cuda.synchronize()
+    return h
+
+
+def _bits(a, b):
+    import torch
+    return torch.equal(a.cpu().view(torch.uint8), b.cpu().view(torch.uint8))
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, TRIP + 5, 32 * TRIP, 32 * TRIP + 1, 70 * TRIP + 1031])
+@pytest.mark.parametrize("gdt,pdt", [("bfloat16", "bfloat16"), ("float16", "float16"), ("float32", None)])
+def test_pinned_state_gives_the_bits_of_device_state(gpu, n, gdt, pdt):
+    import torch
+    from distributedspeed_amd import ops
+    _say(f"host state n={n} {gdt}")
+    gdt, pdt = getattr(torch, gdt), getattr(torch, pdt) if pdt else None
+    p, m, v, p16, g = _inputs(n, gdt, pdt, gpu, n)
+    host = [_pinned(t) for t in (p, m, v)]
+    o16 = p16.clone() if p16 is not None else None
+    ops.adamw_host_state(*host, o16, g, _scalars(gpu, skip=1))  # moves nothing
+    torch.cuda.synchronize()
+    assert all(_bits(h, t) for h, t in zip(host, (p, m, v)))
+    ops.adamw_host_state(*host, o16, g, _scalars(gpu))
+    ops.adamw_flat(p, m, v, p16, g, _scalars(gpu))
+    torch.cuda.synchronize()
+    for name, h, t in zip(("master", "exp_avg", "exp_avg_sq"), host, (p, m, v)):
+        assert _bits(h, t), name
+    assert p16 is None or _bits(o16, p16)
+
+
+@pytest.mark.parametrize("pinned", [True, False])
+def test_the_streamer_takes_pinned_and_pageable_state(gpu, pinned):
+    import torch
+    from distributedspeed_amd import _lib, ops
+    from distributedspeed_amd.offload import HostStateStreamer
+    n, cut = 100_040, 40_008
+    p, m, v, p16, g = _inputs(n, torch.bfloat16, torch.bfloat16, gpu, 3)
+    host = [_pinned(t) if pinned else t.cpu() for t in (p, m, v)]
+    o16 = p16.clone()
+    if not pinned:
+        with pytest.raises(_lib.DsxError, match="not pinned"):
+            ops.adamw_host_state(*host, o16, g, _scalars(gpu))
+    st = HostStateStreamer(gpu, 8192)
+    first, second = torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)
+    for s in (first, second):  # two steps on two streams, in order
+        s.wait_stream(torch.cuda.current_stream(gpu))
+        s.wait_stream(first)
+        with torch.cuda.stream(s):
+            st.run(tuple(host), o16, g, [(0, cut, _scalars(gpu)), (cut, n, _scalars(gpu))])
+    for _ in range(2):
+        ops.adamw_flat(p, m, v, p16, g, _scalars(gpu))
+    torch.cuda.synchronize()
+    assert st.last_bytes == 24 * n
+    for name, h, t in zip(("master", "exp_avg", "exp_avg_sq"), host, (p, m, v)):
+        assert _bits(h, t), name
+    assert _bits(o16, p16)
