@@ -700,7 +700,7 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
         if table is not self._plans_for:  # rebuilt after storage moved: bind again
             st = self.store
             self._k1 = ops.plan_unscale_norm_multi(table, self.dstate, self.partials, self.nparts)
-            k3_table = st.small_table if st.k2_tensors else table
+            k3_table = st.small_table if st.k2_tensors or st.small_table is not None else table
             self._k3 = ops.plan_adamw_multi(k3_table, self.scalars) if k3_table is not None else None
             # K2 per large tensor: everything but the grad is bound here; the
             # grad's address is read at each step (autograd's grads move).
@@ -713,10 +713,10 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
                               st.master[i].numel(), base + ops.SCALARS_BYTES * st.group_of[i])
                              for i in st.k2_tensors]
             self._k2_meta = (pdt, gdt)
-            # The whole step in one call (dsx_zero_step_multi) when no tensor
-            # goes through K2: its fixed arguments, bound once per table.
+            # The whole step in one call (dsx_zero_step_multi) when one table
+            # serves K1 and K3: its fixed arguments, bound once per table.
             self._one_call = None
-            if not st.k2_tensors:
+            if k3_table is table:
                 self._one_call = (_lib.load().dsx_zero_step_multi,
                                   (ops._ptr(table.tensors), ops._ptr(table.chunks), ctypes.c_int64(table.nchunks),
                                    ctypes.c_int64(table.numel), table.pdt, table.gdt, ops._ptr(self.dstate)),

@@ -5,10 +5,10 @@ parameter's grad as its own tensor and steps them one by one (torch
 AdamW's per-tensor loop, Src/zero/stage1.py:522-525); here every parameter
 keeps its own storage and its own autograd-allocated grad, and the step runs
 over the list through a device chunk table (dsx_unscale_norm_multi /
-dsx_adamw_multi): one launch each for the norm and the update whatever the
-number of tensors. When the list falls in K3's one-block-per-CU range, its
-tensors of at least K2_TENSOR_ELEMS elements step through K2
-(dsx_adamw_flat) one by one instead, and K3 takes the rest.
+dsx_adamw_multi): a few launches for the norm and the update whatever the
+number of tensors. In a mid-size list the tensors of at least K2_TENSOR_ELEMS
+elements step through K2 (dsx_adamw_flat) one by one instead, and K3 takes
+the rest.
 
 Per parameter: master / exp_avg / exp_avg_sq are fp32 tensors of the
 parameter's shape owned here; with a 16-bit param dtype, param.data is the
@@ -23,15 +23,21 @@ import torch
 from . import ops
 
 
-# Tensors of at least this many elements step through K2 one by one (the
-# rest through K3) when the whole list would put K3 in its one-block-per-CU
-# regime (K3_SPLIT_RANGE chunks per CU). Measured on MI355X: a 12-layer Llama
-# list (2.9e9 elements, 174 chunks per CU) 15.66 -> 13.64 ms; configs[1]'s
-# GPT-2-small list (30 per CU) 0.6437 -> 0.6404 ms; configs[3]'s list (496
-# per CU, K3's many-blocks regime) is faster as one K3 launch (37.72 against
-# 38.72 ms) and stays so.
+# Mid-size lists, up to K3_MANY_PER_CU chunks per CU, step their tensors of at
+# least K2_TENSOR_ELEMS elements through K2 one by one and the rest through K3
+# over a table of its own in small chunks (k3_chunk_elems); smaller lists, up
+# to K3_SMALL_PER_CU chunks of at most 4096 elements per CU, are one launch of
+# K3 in its one-chunk-per-block shape, larger ones K3 in its many-blocks shape.
+# Measured on MI355X, update alone: eight tensors of 1.7e7 elements (16 chunks
+# of 32768 per CU) 725 us as one K3 launch in that table, 627 through K2, 628
+# through K3 in 4096-element chunks; a Llama-3-8B layer (2.4e8) 1131 through
+# K2, 1155 through K3; 1.0e9 elements in 60 uneven tensors 4740 with K2 from
+# 2**24 on, 4858 through K3 alone; GPT-2-small (1.24e8, only wte through K2) 608
+# either way; configs[3]'s list (496 chunks per CU) is faster as one K3 launch
+# (37.72 against 38.72 ms).
 K2_TENSOR_ELEMS = 1 << 24
-K3_SPLIT_RANGE = (20, 256)
+K3_SMALL_PER_CU = 20
+K3_MANY_PER_CU = 256
 
 
 def auto_chunk_elems(numel: int) -> int:
@@ -57,17 +63,14 @@ def auto_chunk_elems(numel: int) -> int:
 
 
 def k3_chunk_elems(numel: int) -> int:
-    """Chunk size of K3's own table when a list's large tensors step through
-    K2: a power of two from 65536 down to 4096 that gives at least 16384
-    chunks where possible. What K3 then takes is many mid-size and small
-    tensors (configs[1]'s 147 GPT-2-small tensors besides wte: 85.8e6
-    elements), which it runs faster in small chunks: on two MI355X boxes, in
-    one process each, 4096-element chunks against the 16384 of
-    auto_chunk_elems took 407 against 414 us and 429 against 463 us (the
-    whole 148-tensor list: 613 against 641 us)."""
-    c = 65536
-    while c > 4096 and numel // c < 16384:
-        c //= 2
+    """Chunk size of K3's own table over what a mid-size list leaves to K3:
+    4096 (1.34e8 elements in 4096 / 8192 / 16384 / 32768 / 65536-element chunks:
+    628 / 626 / 655 / 687 / 691 us, the GPT-2-small list in the first three 608 /
+    617 / 650), larger only to stay clear of K3's many-blocks shape (256 chunks
+    per CU), which is for 65536-element chunks."""
+    c = 4096
+    while c < 65536 and numel // c > 60000:
+        c *= 2
     return c
 
 
@@ -112,11 +115,12 @@ class RaggedParams:
                         p.grad = p.grad.to(self.device, self.grad_dtype).contiguous()
         self.numel = sum(m.numel() for m in self.master)
         self.chunk_elems = int(chunk_elems) if chunk_elems else auto_chunk_elems(self.numel)
+        self._own_chunks = bool(chunk_elems)
         self.ngroups = len(groups)
         self._table = None
         self._key = None
         self.k2_tensors: list[int] = []  # tensors the step runs through K2 (decided with each table)
-        self.small_table = None  # K3's table over the other tensors when k2_tensors is not empty
+        self.small_table = None  # K3's own table over the other tensors, where it has one
 
     def ensure_grads(self) -> None:
         """Give every param a contiguous grad of the grad dtype on the device
@@ -164,7 +168,9 @@ class RaggedParams:
         cus = torch.cuda.get_device_properties(self.device).multi_processor_count
         per_cu = self._table.nchunks / cus
         big = []
-        if K3_SPLIT_RANGE[0] <= per_cu < K3_SPLIT_RANGE[1]:
+        small = per_cu < K3_SMALL_PER_CU and (self._own_chunks or self.chunk_elems <= 4096)
+        mid = not small and per_cu < K3_MANY_PER_CU
+        if mid:
             # K2 needs every array 16-byte aligned. master / exp_avg / exp_avg_sq
             # are allocated here and ensure_grads realigns a large tensor's grad
             # before each step, but param.data may have been replaced by a
@@ -177,13 +183,14 @@ class RaggedParams:
         taken = set(big)
         self._small = [i for i in range(len(self.params)) if i not in taken]
         self.small_table = None
-        if big and self._small:
-            sub = self._small
-            n_small = sum(self.master[i].numel() for i in sub)
+        sub = self._small
+        n_small = sum(self.master[i].numel() for i in sub)
+        c = k3_chunk_elems(n_small)
+        if sub and (big or (mid and not self._own_chunks and c < self.chunk_elems)):
             self.small_table = ops.ChunkTable(
                 [self.master[i] for i in sub], [self.exp_avg[i] for i in sub], [self.exp_avg_sq[i] for i in sub],
                 None if p16 is None else [p16[i] for i in sub], [self.params[i].grad for i in sub],
-                [self.group_of[i] for i in sub], k3_chunk_elems(n_small))
+                [self.group_of[i] for i in sub], c)
 
     def zero_grad(self, set_to_none: bool = False) -> None:
         """set_to_none: p.grad = None, so the next backward's grads are read

@@ -1,0 +1,84 @@
+"""K3's launch shapes by chunk count (one chunk per block, one block per CU in
+one launch and in several, many blocks) and the tables the ragged store builds
+for mid-size lists: the same bits as K2 over the same elements."""
+from __future__ import annotations
+
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(msg):
+    print(f"[gpu-test] {msg}", file=sys.stderr, flush=True)
+
+
+def _bits(a, b):
+    import torch
+    return torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+
+
+# chunks per CU around each change of shape, and chunks past a multiple of 256
+@pytest.mark.parametrize("per_cu,extra", [(1, -1), (20, 0), (20, 1), (64, 0), (64, 1), (129, 77), (256, -1), (256, 3)])
+@pytest.mark.parametrize("gdt", ["bfloat16", "float32"])
+def test_every_k3_shape_gives_k2s_bits(gpu, per_cu, extra, gdt):
+    import torch
+    from distributedspeed_amd import ops
+    from distributedspeed_amd._lib import DsxStepScalars
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    nchunks, chunk = per_cu * cus + extra, 24
+    gdt = getattr(torch, gdt)
+    pdt = torch.bfloat16 if gdt == torch.bfloat16 else None
+    n = nchunks * chunk - 8  # the last chunk of the last tensor is short
+    _say(f"K3 shape chunks={nchunks} {gdt}")
+    gen = torch.Generator(device=gpu).manual_seed(per_cu)
+    p, m = (torch.empty(n, device=gpu).normal_(0.0, 0.02, generator=gen) for _ in range(2))
+    v = torch.empty(n, device=gpu).uniform_(0.0, 1e-6, generator=gen)
+    g = torch.empty(n, device=gpu).normal_(0.0, 1e-3, generator=gen).to(gdt)
+    p16 = p.to(pdt) if pdt else None
+    cuts = [0, chunk, (nchunks // 2) * chunk, n]
+
+    def split(t):
+        return [t[a:b].clone() for a, b in zip(cuts, cuts[1:])] if t is not None else None
+
+    sp, sm, sv, s16, sg = (split(t) for t in (p, m, v, p16, g))
+    table = ops.ChunkTable(sp, sm, sv, s16, sg, chunk_elems=chunk)
+    assert table.nchunks == nchunks
+    sc = DsxStepScalars()
+    sc.inv_scale, sc.clip_coef, sc.decay, sc.w1, sc.w1c = 1.0, 0.5, 0.9999, 0.1, 0.9
+    sc.b2, sc.val2, sc.eps, sc.bc2s, sc.nss = 0.999, 0.001, 1e-8, 0.3, -1e-3
+    scal = ops.scalars_from_host(sc, gpu)
+    ops.adamw_multi(table, scal)
+    ops.adamw_flat(p, m, v, p16, g, scal)
+    for name, got, ref in (("master", sp, p), ("exp_avg", sm, m), ("exp_avg_sq", sv, v), ("param16", s16, p16)):
+        assert got is None or _bits(torch.cat(got), ref), name
+
+
+# chunks of 8192 (16-20 and 20-32 per CU) without and with tensors of K2's
+# size, and a list of K2's tensors alone
+@pytest.mark.parametrize("sizes,big", [((13_000_008, 9_000_001, 14_000_000), 0), ((15_000_000, 16_500_000, 16_000_003), 0),
+                                       ((17_000_000, 20_000_000, 77), 2), ((18_000_000, 17_000_000), 2)])
+def test_mid_size_lists_match_the_flat_form(gpu, sizes, big):
+    import torch
+    from distributedspeed_amd.optimizers import AdamWOptimizer, MultiTensorAdamWOptimizer
+    _say(f"mid-size list {sizes}")
+    gen = torch.Generator(device=gpu).manual_seed(5)
+    init = [torch.empty(k, device=gpu).normal_(0.0, 0.02, generator=gen) for k in sizes]
+    grads = [torch.empty(k, device=gpu).normal_(0.0, 1e-3, generator=gen).to(torch.bfloat16) for k in sizes]
+    opts = []
+    for cls in (AdamWOptimizer, MultiTensorAdamWOptimizer):
+        ps = [torch.nn.Parameter(t.clone()) for t in init]
+        opt = cls(ps, lr=1e-3, param_dtype=torch.bfloat16, device=gpu, max_grad_norm=1.0)
+        for _ in range(2):
+            for p, g in zip(ps, grads):
+                p.grad = g.clone()
+            opt.step()
+        opts.append((ps, opt))
+    store = opts[1][1].store
+    assert store.chunk_elems == 8192 and len(store.k2_tensors) == big
+    assert (store.small_table is None) == (big == len(sizes))
+    for pf, pr in zip(opts[0][0], opts[1][0]):
+        assert _bits(pf.data, pr.data)
+        for key in ("master", "exp_avg", "exp_avg_sq"):
+            assert _bits(opts[0][1].state[pf][key], opts[1][1].state[pr][key]), key
