@@ -99,6 +99,7 @@ constexpr int64_t kK2LargeN = int64_t(3) << 27;  // K2's large-partition shape f
 constexpr int64_t kMaxGridBlocks = int64_t(1) << 22;  // 2^30 work-items of kBlock threads
 constexpr int64_t kK2OneTripPerCu = 32;  // K2's one-trip grid up to this many blocks per CU
 constexpr int64_t kK3OneChunkPerCu = 20;  // K3: one chunk per block up to this many chunks per CU
+constexpr int64_t kK3FoldChunksPerCu = 24;  // K3 with K0 folded in up to this many chunks per CU
 constexpr int64_t kK3PartPerCu = 64;      // K3, one block per CU: at most this many chunks per CU a launch
 
 struct Tuning {
@@ -154,6 +155,11 @@ int64_t ceil_div(int64_t a, int64_t b) { return a / b + (a % b > 0 ? 1 : 0); }
 
 template <bool NT, typename T>
 __device__ __forceinline__ T ld(const T* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool NT, typename T>
+__device__ __forceinline__ T ld(const T __attribute__((address_space(1))) * p) {
   if constexpr (NT) return __builtin_nontemporal_load(p);
   else return *p;
 }
@@ -1011,7 +1017,51 @@ __device__ __forceinline__ Sc uniform_sc(const Sc& a) {
 __device__ __forceinline__ const DsxGroupsDev& group_block(const DsxGroupsDev& g) { return g; }
 __device__ __forceinline__ const DsxGroupsDev& group_block(const DsxGroupsDev* g) { return *g; }
 
-template <int GD, int PD, int U, bool NT, typename GB>
+// What the folded kernels leave in the memory-side cache (K1's plain loads have
+// put the grads there). kFoldStream, for the first part of a large partition:
+// every access nontemporal. kFoldSmall: the grads' loads plain, which is
+// 1-5% faster while they are few (flat steps on MI355X, three states in turn,
+// us: 1.9e6 fp16 elements 14.7 -> 13.9, 7.1e6 bf16 39.9 -> 39.3, 1.6e7 79.8 ->
+// 79.2; from 9e7 on slower, 428 -> 436). kFoldKeep, while the fp32 state is at
+// most kKeepStateBytes: the stores are also written through to the
+// memory-side cache (scope bit sc1) instead of past it, so that the next step's
+// loads find the state there if what ran in between has not displaced it, and
+// no dirty lines are left in the L2s for the kernel's end to write back (plain
+// stores: 14.4 against 12.6 us at 1.9e6 elements). us with three states in turn
+// / one state again and again, kFoldSmall against kFoldKeep: 1.9e6 elements
+// 13.9 / 11.2 against 12.6 / 12.0, 2.5e6 18.0 / 15.3 against 15.6 / 14.8, 4.0e6
+// 25.1 / 23.7 against 22.4 / 21.6, 5.0e6 30.1 / 28.5 against 27.1 / 26.0; from
+// 7.1e6 on only one state alone gains (39.3 / 38.7 against 40.1 / 34.9, 1.6e7
+// 79.2 / 78.6 against 82.0 / 72.9), which a training step in between would
+// displace. kFoldPlain: the nontemporal hint switched off.
+enum FoldPolicy { kFoldPlain = 0, kFoldStream = 1, kFoldSmall = 2, kFoldKeep = 3 };
+constexpr int64_t kKeepStateBytes = int64_t(1) << 26;
+
+// Where a folded kernel stores one array's slots (n of them from p on; for
+// kFoldKeep n * sizeof(T) fits 31 bits, as kKeepStateBytes does).
+template <typename T, int POL>
+struct Slots {
+  T* p;
+  __device__ __forceinline__ Slots(T* base, int64_t) : p(base) {}
+  __device__ __forceinline__ void put(int64_t i, const T& x) const { st<POL != kFoldPlain>(p + i, x); }
+};
+
+template <typename T>
+struct Slots<T, kFoldKeep> {
+  static constexpr int kRawBuffer = 0x00027000;  // untyped, bounds-checked
+  static constexpr int kSc1 = 16;
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ Slots(T* base, int64_t n)
+      : r(__builtin_amdgcn_make_buffer_rsrc(base, 0, (int)(n * (int64_t)sizeof(T)), kRawBuffer)) {}
+  __device__ __forceinline__ void put(int64_t i, const T& x) const {
+    if constexpr (sizeof(T) == 16)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, (int)(i * 16), 0, kSc1);
+    else
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), r, (int)(i * 8), 0, kSc1);
+  }
+};
+
+template <int GD, int PD, int U, int POL, typename GB>
 __global__ __launch_bounds__(kBlock) void k2_adamw_fold(float* __restrict__ p, float* __restrict__ m,
                                                         float* __restrict__ v, uint16_t* __restrict__ p16,
                                                         const void* __restrict__ gv, int64_t n,
@@ -1019,6 +1069,7 @@ __global__ __launch_bounds__(kBlock) void k2_adamw_fold(float* __restrict__ p, f
                                                         DsxState* state, DsxScalerConfig scfg, GB gb,
                                                         int32_t max_groups, int32_t group, int32_t writer,
                                                         DsxStepScalars* __restrict__ out) {
+  constexpr bool NT = POL != kFoldPlain;
   constexpr bool DEV = std::is_pointer<GB>::value;
   const DsxGroupsDev& grp = group_block(gb);
   const bool groups_bad = DEV ? groups_bad_dev(grp, max_groups) : false;
@@ -1074,13 +1125,15 @@ __global__ __launch_bounds__(kBlock) void k2_adamw_fold(float* __restrict__ p, f
   const int64_t nvec = n >> 2;
   const int64_t stride = (int64_t)(gridDim.x - (writer ? 1 : 0)) * kBlock * U;  // the slot blocks
   int64_t i0 = (int64_t)blockIdx.x * kBlock * U + threadIdx.x;
+  const Slots<f4, POL> sp(p4, nvec), sm(m4, nvec), sv(v4, nvec);
+  const Slots<u2, POL> so(o2, cast ? nvec : 0);
   GS Gs[U];
   f4 P[U], M[U], V[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     int64_t i = i0 + (int64_t)u * kBlock;
     i = i < nvec ? i : nvec - 1;  // nvec >= 1 (n >= 4 on this path)
-    Gs[u] = ld<NT>(g4 + i);
+    Gs[u] = ld<POL == kFoldStream>(g4 + i);
     P[u] = ld<NT>(p4 + i);
     M[u] = ld<NT>(m4 + i);
     V[u] = ld<NT>(v4 + i);
@@ -1123,10 +1176,10 @@ __global__ __launch_bounds__(kBlock) void k2_adamw_fold(float* __restrict__ p, f
         G::four(Gs[u], gf);
         f4 pp = P[u], mm = M[u], vv = V[u];
         adamw4(gf, pp, mm, vv, sc);
-        st<NT>(p4 + i, pp);
-        st<NT>(m4 + i, mm);
-        st<NT>(v4 + i, vv);
-        if (cast) st<NT>(o2 + i, pack4<PD>(pp));
+        sp.put(i, pp);
+        sm.put(i, mm);
+        sv.put(i, vv);
+        if (cast) so.put(i, pack4<PD>(pp));
       }
     }
     slot_loop<GD, PD, U, NT, false, true>(p4, m4, v4, o2, g4, nvec, i0 + stride, stride, sc);
@@ -1293,19 +1346,21 @@ struct Trip {
 // table: device allocations start on 256-byte boundaries, so that stays in
 // the table's allocation; the values go unused), so that the waits for them
 // stay exact.
-template <int GD, int U, bool NT>
+template <int GD, int U, bool GNT, bool NT>
 __device__ __forceinline__ void first_trip(const ChunkView<GD>& c, const void* spare_any, Trip<GD, U>& T) {
   using GS = typename Grad<GD>::slot4;
-  const void* spare = reinterpret_cast<const void*>(reinterpret_cast<uintptr_t>(spare_any) & ~uintptr_t(15));
-  const f4* lp = c.vec ? reinterpret_cast<const f4*>(c.p) : static_cast<const f4*>(spare);
-  const f4* lm = c.vec ? reinterpret_cast<const f4*>(c.m) : static_cast<const f4*>(spare);
-  const f4* lv = c.vec ? reinterpret_cast<const f4*>(c.v) : static_cast<const f4*>(spare);
-  const GS* lg = c.vec ? reinterpret_cast<const GS*>(c.g) : static_cast<const GS*>(spare);
+  typedef const f4 __attribute__((address_space(1)))* F4;  // global loads: vmcnt alone
+  typedef const GS __attribute__((address_space(1)))* G4;
+  const uintptr_t spare = reinterpret_cast<uintptr_t>(spare_any) & ~uintptr_t(15);
+  const F4 lp = (F4)(c.vec ? reinterpret_cast<uintptr_t>(c.p) : spare);
+  const F4 lm = (F4)(c.vec ? reinterpret_cast<uintptr_t>(c.m) : spare);
+  const F4 lv = (F4)(c.vec ? reinterpret_cast<uintptr_t>(c.v) : spare);
+  const G4 lg = (G4)(c.vec ? reinterpret_cast<uintptr_t>(c.g) : spare);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     int64_t i = (int64_t)threadIdx.x + (int64_t)u * kBlock;
     i = !c.vec ? 0 : (i < c.nvec ? i : c.nvec - 1);
-    T.g[u] = ld<NT>(lg + i);
+    T.g[u] = ld<GNT>(lg + i);
     T.p[u] = ld<NT>(lp + i);
     T.m[u] = ld<NT>(lm + i);
     T.v[u] = ld<NT>(lv + i);
@@ -1370,20 +1425,26 @@ __global__ __launch_bounds__(kBlock) void k2_adamw_multi(const DsxTensorRef* __r
 // K1 over the list launched with fold): every block reduces the partials in
 // K0's order and decides the step with K0's code on the entry values, then
 // steps its chunk with its group's scalars; the last block does no chunk
-// work and writes the step records and the state's updated fields. One
-// chunk per block (the small-list shape: the grid is the chunk count and the
-// writer); 1 <= nparts <= kFoldMaxParts.
-template <int GD, int PD, bool NT>
+// work and writes the step records and the state's updated fields. The
+// small-list shape: `split` blocks per chunk, each with one of its spans of
+// whole trips, so that a span is one trip (4096-element chunks in two spans
+// against one block each, us a step, the flat form in brackets: 2.5e6 elements
+// 16.5 / 21.1 [15.7], 4.0e6 23.7 / 26.1 [22.8], 7.0e6 39.6 / 42.2 [38.8], 1.6e7
+// 80.7 / 86.3 [79.9]);
+// the grid is nchunks * split and the writer; 1 <= nparts <= kFoldMaxParts.
+template <int GD, int PD, int POL>
 __global__ __launch_bounds__(kBlock) void k3_adamw_fold(const DsxTensorRef* __restrict__ tensors,
-                                                        const DsxChunk* __restrict__ chunks, int64_t nchunks,
+                                                        const DsxChunk* __restrict__ chunks, int64_t nchunks, int32_t split,
                                                         const double* __restrict__ partials, int32_t nparts,
                                                         DsxState* state, DsxScalerConfig scfg, DsxGroupsDev grp,
                                                         DsxStepScalars* __restrict__ out) {
   constexpr int U = 2;
-  // The host launches nchunks + 1 blocks: one per chunk, then the writer (a
-  // larger grid's extra blocks would return here).
-  if ((int64_t)blockIdx.x > nchunks) return;
-  if ((int64_t)blockIdx.x == nchunks) {
+  constexpr bool NT = POL != kFoldPlain;
+  // The host launches nchunks * split + 1 blocks: the chunks' spans, then the
+  // writer (a larger grid's extra blocks would return here).
+  const int64_t spans = nchunks * split;
+  if ((int64_t)blockIdx.x > spans) return;
+  if ((int64_t)blockIdx.x == spans) {
     double x = 0.0;
     for (int i = threadIdx.x; i < nparts; i += kBlock) x += partials[i];  // reduce_partials' order
     const double sumsq = block_sum_all(x);
@@ -1419,11 +1480,19 @@ __global__ __launch_bounds__(kBlock) void k3_adamw_fold(const DsxTensorRef* __re
     const double x = partials[i < nparts ? i : nparts - 1];
     pv[j] = i < nparts ? x : 0.0;
   }
-  const DsxChunk ch = chunk_rec(chunks, blockIdx.x);  // < nchunks: nchunks slot blocks and the writer
+  DsxChunk ch = chunk_rec(chunks, blockIdx.x / (uint32_t)split);  // < nchunks: the spans' blocks
+  if (split > 1) {  // this block's span: whole trips, the last one what is left (perhaps nothing)
+    constexpr int64_t kTrip = (int64_t)kBlock * U * 4;
+    const int64_t span = (ch.len + kTrip * split - 1) / (kTrip * split) * kTrip;
+    const int64_t at = span * (blockIdx.x % (uint32_t)split);
+    if (at >= ch.len) return;
+    ch.start += at;
+    ch.len = ch.len - at < span ? ch.len - at : span;
+  }
   const DsxTensorRef tr = tensor_rec(tensors, ch.tensor);
   const ChunkView<GD> cv = chunk_view<GD>(tr, ch);
   Trip<GD, U> T;
-  first_trip<GD, U, NT>(cv, tensors, T);
+  first_trip<GD, U, POL == kFoldStream, NT>(cv, tensors, T);
   asm volatile("" ::: "memory");  // the slot loads issue here
   asm volatile("" : "+v"(t2), "+v"(scale0), "+v"(coef1));
   DsxState s = {};
@@ -1443,6 +1512,10 @@ __global__ __launch_bounds__(kBlock) void k3_adamw_fold(const DsxTensorRef* __re
   if (d.skip || tr.group >= d.ng) return;
   const Sc sc = uniform_sc(load_sc(record_bc(d, s, grp, tr.group, sumsq, bc1, bc2s)));
   if (cv.vec) {
+    const int64_t trip = cv.nvec < U * kBlock ? cv.nvec : U * kBlock;  // in 31 bits whatever the chunk
+    const Slots<f4, POL> sp(reinterpret_cast<f4*>(cv.p), trip), sm(reinterpret_cast<f4*>(cv.m), trip),
+        sv(reinterpret_cast<f4*>(cv.v), trip);
+    const Slots<u2, POL> so(reinterpret_cast<u2*>(cv.p16), cv.p16 ? trip : 0);
     // As in k2_adamw_fold: the first trip's loads taken in on every path.
 #pragma unroll
     for (int u = 0; u < U; ++u) asm volatile("" : "+v"(T.g[u]), "+v"(T.p[u]), "+v"(T.m[u]), "+v"(T.v[u]));
@@ -1454,10 +1527,10 @@ __global__ __launch_bounds__(kBlock) void k3_adamw_fold(const DsxTensorRef* __re
         Grad<GD>::four(T.g[u], gf);
         f4 pp = T.p[u], mm = T.m[u], vv = T.v[u];
         adamw4(gf, pp, mm, vv, sc);
-        st<NT>(reinterpret_cast<f4*>(cv.p) + i, pp);
-        st<NT>(reinterpret_cast<f4*>(cv.m) + i, mm);
-        st<NT>(reinterpret_cast<f4*>(cv.v) + i, vv);
-        if (cv.p16) st<NT>(reinterpret_cast<u2*>(cv.p16) + i, pack4<PD>(pp));
+        sp.put(i, pp);
+        sm.put(i, mm);
+        sv.put(i, vv);
+        if (cv.p16) so.put(i, pack4<PD>(pp));
       }
     }
     chunk_slots<GD, PD, U, NT, false>(cv, (int64_t)threadIdx.x + (int64_t)kBlock * U, sc);
@@ -1707,23 +1780,23 @@ struct FoldGroups {
 // The folded K2 over one group's range: the one-trip grid of K2 (2 slots per
 // thread, at most kK2OneTripPerCu blocks per CU; the kernel strides over what
 // one trip does not cover), plus the writer's block.
-template <int GD, int PD, bool NT>
-void launch_k2_fold_nt(dim3 grid, float* p, float* m, float* v, uint16_t* o, const void* g, int64_t n,
+template <int GD, int PD, int POL>
+void launch_k2_fold_pol(dim3 grid, float* p, float* m, float* v, uint16_t* o, const void* g, int64_t n,
                        const double* partials, int32_t nparts, DsxState* state, const DsxScalerConfig& scfg,
                        const FoldGroups& fg, int group, int32_t w, DsxStepScalars* out, hipStream_t s) {
   constexpr int U = 2;
   if (fg.dev)
-    hipLaunchKernelGGL((k2_adamw_fold<GD, PD, U, NT, const DsxGroupsDev*>), grid, dim3(kBlock), 0, s, p, m, v, o, g,
+    hipLaunchKernelGGL((k2_adamw_fold<GD, PD, U, POL, const DsxGroupsDev*>), grid, dim3(kBlock), 0, s, p, m, v, o, g,
                        n, partials, nparts, state, scfg, fg.dev, fg.max_groups, group, w, out);
   else
-    hipLaunchKernelGGL((k2_adamw_fold<GD, PD, U, NT, DsxGroupsDev>), grid, dim3(kBlock), 0, s, p, m, v, o, g, n,
+    hipLaunchKernelGGL((k2_adamw_fold<GD, PD, U, POL, DsxGroupsDev>), grid, dim3(kBlock), 0, s, p, m, v, o, g, n,
                        partials, nparts, state, scfg, *fg.host, fg.max_groups, group, w, out);
 }
 
 template <int GD, int PD>
 void launch_k2_fold(float* p, float* m, float* v, void* p16, const void* g, int64_t n, const double* partials,
                     int32_t nparts, DsxState* state, const DsxScalerConfig& scfg, const FoldGroups& fg,
-                    int group, bool writer, DsxStepScalars* out, hipStream_t s, int64_t blocks_per_cu) {
+                    int group, bool writer, DsxStepScalars* out, hipStream_t s, int64_t blocks_per_cu, int pol) {
   const int64_t slots = n >> 2;
   int64_t blocks = ceil_div(slots > 0 ? slots : 1, (int64_t)kBlock * 2);
   const int64_t cap = (int64_t)cu_count() * blocks_per_cu;
@@ -1732,21 +1805,26 @@ void launch_k2_fold(float* p, float* m, float* v, void* p16, const void* g, int6
   uint16_t* o = static_cast<uint16_t*>(p16);
   const dim3 grid((unsigned)blocks);
   const int32_t w = writer ? 1 : 0;
-  if (g_tune.nontemporal)
-    launch_k2_fold_nt<GD, PD, true>(grid, p, m, v, o, g, n, partials, nparts, state, scfg, fg, group, w, out, s);
-  else
-    launch_k2_fold_nt<GD, PD, false>(grid, p, m, v, o, g, n, partials, nparts, state, scfg, fg, group, w, out, s);
+#define DSX_FOLD(POL) \
+  launch_k2_fold_pol<GD, PD, POL>(grid, p, m, v, o, g, n, partials, nparts, state, scfg, fg, group, w, out, s)
+  switch (pol) {
+    case kFoldPlain: DSX_FOLD(kFoldPlain); break;
+    case kFoldStream: DSX_FOLD(kFoldStream); break;
+    case kFoldSmall: DSX_FOLD(kFoldSmall); break;
+    default: DSX_FOLD(kFoldKeep); break;
+  }
+#undef DSX_FOLD
 }
 
 template <int GD>
 void k2_fold_by_param(int pd, float* p, float* m, float* v, void* p16, const void* g, int64_t n,
                       const double* partials, int32_t nparts, DsxState* state, const DsxScalerConfig& scfg,
                       const FoldGroups& fg, int group, bool writer, DsxStepScalars* out, hipStream_t s,
-                      int64_t bpc) {
+                      int64_t bpc, int pol) {
   if (pd == DSX_BF16)
-    launch_k2_fold<GD, DSX_BF16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, bpc);
+    launch_k2_fold<GD, DSX_BF16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, bpc, pol);
   else
-    launch_k2_fold<GD, DSX_F16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, bpc);
+    launch_k2_fold<GD, DSX_F16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, bpc, pol);
 }
 
 bool fold_applies(int64_t n, int32_t nparts) {
@@ -1769,25 +1847,34 @@ int64_t k2_first_part(int64_t n) {
   return ceil_div(ceil_div(n, ceil_div(n, want)), 1024) * 1024;
 }
 
+// The folded kernels' policy for a step over n elements.
+int fold_policy(int nontemporal, int64_t n) {
+  if (!nontemporal) return kFoldPlain;
+  if (n > g_tune.fold_max_elems) return kFoldStream;
+  return n <= kKeepStateBytes / 12 ? kFoldKeep : kFoldSmall;
+}
+
 // The folded K2 over n elements: K2's one-trip grid (at most
-// kK2OneTripPerCu blocks per CU), or at most bpc blocks per CU.
+// kK2OneTripPerCu blocks per CU), or at most bpc blocks per CU. step_elems: the
+// elements of the whole step, by which the policy is chosen.
 int do_adamw_fold(float* p, float* m, float* v, void* p16, int pdt, const void* g, int gdt, int64_t n,
                   const double* partials, int32_t nparts, DsxState* state, const DsxScalerConfig& scfg,
                   const FoldGroups& fg, int group, bool writer, DsxStepScalars* out, hipStream_t s,
-                  int64_t bpc = kK2OneTripPerCu) {
+                  int64_t step_elems, int64_t bpc = kK2OneTripPerCu) {
   const int pd = p16 ? pdt : DSX_F16;
+  const int pol = fold_policy(g_tune.nontemporal, step_elems);
   switch (gdt) {
     case DSX_BF16:
       k2_fold_by_param<DSX_BF16>(pd, p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s,
-                                 bpc);
+                                 bpc, pol);
       break;
     case DSX_F16:
       k2_fold_by_param<DSX_F16>(pd, p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s,
-                                bpc);
+                                 bpc, pol);
       break;
     default:
       k2_fold_by_param<DSX_F32>(pd, p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s,
-                                bpc);
+                                 bpc, pol);
       break;
   }
   return launch_status("dsx_adamw_flat (finalize folded in)");
@@ -1885,14 +1972,14 @@ int zero_step_flat(float* master, float* m, float* v, void* p16, int pdt, const 
   if (fold_applies(n, nparts)) {
     int rc = do_unscale_norm(g, gdt, n, state, partials, nparts, s, state);
     if (!rc) rc = do_adamw_fold(master, m, v, p16, pdt, g, gdt, n, partials, nparts, state, scaler,
-                                FoldGroups{&grp, nullptr, 1}, 0, true, out, s);
+                                FoldGroups{&grp, nullptr, 1}, 0, true, out, s, n);
     return rc;
   }
   if (fold_first_applies(n, nparts)) {
     const int64_t a = k2_first_part(n);
     int rc = do_unscale_norm(g, gdt, n, state, partials, nparts, s, state);
     if (!rc) rc = do_adamw_fold(master, m, v, p16, pdt, g, gdt, a, partials, nparts, state, scaler,
-                                FoldGroups{&grp, nullptr, 1}, 0, true, out, s, 1);
+                                FoldGroups{&grp, nullptr, 1}, 0, true, out, s, n, 1);
     if (!rc && a < n) {
       void* p16a = p16 ? static_cast<void*>(static_cast<uint16_t*>(p16) + a) : nullptr;
       const void* ga = static_cast<const char*>(g) + a * (gdt == DSX_F32 ? 4 : 2);
@@ -2025,26 +2112,34 @@ int do_adamw_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t 
   return launch_status("dsx_adamw_multi");
 }
 
+template <int GD, int PD>
+void launch_k3_fold_p(int pol, int32_t split, const DsxTensorRef* t, const DsxChunk* c, int64_t nc,
+                      const double* partials, int32_t nparts, DsxState* state, const DsxScalerConfig& scfg,
+                      const DsxGroupsDev& grp, DsxStepScalars* out, hipStream_t s) {
+#define DSX_FOLD(POL) \
+  hipLaunchKernelGGL((k3_adamw_fold<GD, PD, POL>), grid, dim3(kBlock), 0, s, t, c, nc, split, partials, nparts, state, \
+                     scfg, grp, out)
+  const dim3 grid((unsigned)(nc * split + 1));  // the chunks' spans, and the writer
+  switch (pol) {  // a list of the fold's size never streams
+    case kFoldPlain: DSX_FOLD(kFoldPlain); break;
+    case kFoldSmall: DSX_FOLD(kFoldSmall); break;
+    default: DSX_FOLD(kFoldKeep); break;
+  }
+#undef DSX_FOLD
+}
+
 template <int GD>
-void launch_k3_fold(int pd, dim3 grid, const DsxTensorRef* t, const DsxChunk* c, int64_t nc, const double* partials,
+void launch_k3_fold(int pd, int64_t numel, const DsxTensorRef* t, const DsxChunk* c, int64_t nc, const double* partials,
                     int32_t nparts, DsxState* state, const DsxScalerConfig& scfg, const DsxGroupsDev& grp,
                     DsxStepScalars* out, hipStream_t s) {
-  const bool nt = g_tune.k3_nontemporal != 0;
-  if (pd == DSX_BF16) {
-    if (nt)
-      hipLaunchKernelGGL((k3_adamw_fold<GD, DSX_BF16, true>), grid, dim3(kBlock), 0, s, t, c, nc, partials, nparts,
-                         state, scfg, grp, out);
-    else
-      hipLaunchKernelGGL((k3_adamw_fold<GD, DSX_BF16, false>), grid, dim3(kBlock), 0, s, t, c, nc, partials, nparts,
-                         state, scfg, grp, out);
-  } else {
-    if (nt)
-      hipLaunchKernelGGL((k3_adamw_fold<GD, DSX_F16, true>), grid, dim3(kBlock), 0, s, t, c, nc, partials, nparts,
-                         state, scfg, grp, out);
-    else
-      hipLaunchKernelGGL((k3_adamw_fold<GD, DSX_F16, false>), grid, dim3(kBlock), 0, s, t, c, nc, partials, nparts,
-                         state, scfg, grp, out);
-  }
+  // Spans of one trip for chunks of the list's mean length, at most 8.
+  const int64_t trips = ceil_div(ceil_div(numel, nc), (int64_t)kBlock * 2 * 4);
+  const int32_t split = (int32_t)(trips < 1 ? 1 : trips > 8 ? 8 : trips);
+  const int pol = fold_policy(g_tune.k3_nontemporal, numel);
+  if (pd == DSX_BF16)
+    launch_k3_fold_p<GD, DSX_BF16>(pol, split, t, c, nc, partials, nparts, state, scfg, grp, out, s);
+  else
+    launch_k3_fold_p<GD, DSX_F16>(pol, split, t, c, nc, partials, nparts, state, scfg, grp, out, s);
 }
 
 // The flat plan's own checks (everything but the group block).
@@ -2105,13 +2200,13 @@ int plan_launches(const DsxFlatPlan& P, const DsxGroupsDev* G, const DsxGroupsDe
     const void* ga = static_cast<const char*>(P.grad) + a * gsz;
     if (fold) {
       rc = do_adamw_fold(P.master + a, P.exp_avg + a, P.exp_avg_sq + a, p16, P.param_dtype, ga, P.grad_dtype, b - a,
-                         P.partials, P.nparts, P.state, P.scaler, fg, k, writer, P.out, s);
+                         P.partials, P.nparts, P.state, P.scaler, fg, k, writer, P.out, s, P.n);
     } else if (first && writer) {
       // The step's first part decides and writes the records; the rest of
       // this group and the other groups read them.
       const int64_t c = k2_first_part(b - a);
       rc = do_adamw_fold(P.master + a, P.exp_avg + a, P.exp_avg_sq + a, p16, P.param_dtype, ga, P.grad_dtype, c,
-                         P.partials, P.nparts, P.state, P.scaler, fg, k, true, P.out, s, 1);
+                         P.partials, P.nparts, P.state, P.scaler, fg, k, true, P.out, s, P.n, 1);
       if (!rc && c < b - a) {
         void* p16c = p16 ? static_cast<void*>(static_cast<uint16_t*>(p16) + c) : nullptr;
         rc = do_adamw_flat(P.master + a + c, P.exp_avg + a + c, P.exp_avg_sq + a + c, p16c, P.param_dtype,
@@ -2571,9 +2666,9 @@ int dsx_zero_step_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int
     if (G.t_offset[k] < 0) return fail(DSX_EINVAL, "negative t_offset for group %d", k);
   }
   hipStream_t s = as_stream(stream);
-  // Two launches where the fold applies and the list takes K3's one-chunk-
-  // per-block shape; else K1, K0, K3.
-  const bool fold = nchunks > 0 && fold_applies(numel, nparts) && nchunks <= kK3OneChunkPerCu * cu_count();
+  // Two launches where the fold applies (3 * 2^23 elements are 24 chunks of
+  // 4096 per CU) and the list has few chunks; else K1, K0, K3.
+  const bool fold = nchunks > 0 && fold_applies(numel, nparts) && nchunks <= kK3FoldChunksPerCu * cu_count();
   rc = do_unscale_norm_multi(tensors, chunks, nchunks, grad_dtype, state, partials, nparts, s,
                              fold ? state : nullptr);
   if (rc) return rc;
@@ -2582,13 +2677,12 @@ int dsx_zero_step_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int
     if (!rc) rc = do_adamw_multi(tensors, chunks, nchunks, param_dtype, grad_dtype, out, s);
     return rc;
   }
-  const dim3 grid((unsigned)(nchunks + 1));  // one chunk per block, and the writer
   switch (grad_dtype) {
-    case DSX_BF16: launch_k3_fold<DSX_BF16>(param_dtype, grid, tensors, chunks, nchunks, partials, nparts, state,
+    case DSX_BF16: launch_k3_fold<DSX_BF16>(param_dtype, numel, tensors, chunks, nchunks, partials, nparts, state,
                                             scaler, G, out, s); break;
-    case DSX_F16: launch_k3_fold<DSX_F16>(param_dtype, grid, tensors, chunks, nchunks, partials, nparts, state,
+    case DSX_F16: launch_k3_fold<DSX_F16>(param_dtype, numel, tensors, chunks, nchunks, partials, nparts, state,
                                           scaler, G, out, s); break;
-    default: launch_k3_fold<DSX_F32>(param_dtype, grid, tensors, chunks, nchunks, partials, nparts, state, scaler,
+    default: launch_k3_fold<DSX_F32>(param_dtype, numel, tensors, chunks, nchunks, partials, nparts, state, scaler,
                                      G, out, s); break;
   }
   return launch_status("dsx_zero_step_multi (finalize folded in)");

@@ -82,3 +82,45 @@ def test_mid_size_lists_match_the_flat_form(gpu, sizes, big):
         assert _bits(pf.data, pr.data)
         for key in ("master", "exp_avg", "exp_avg_sq"):
             assert _bits(opts[0][1].state[pf][key], opts[1][1].state[pr][key]), key
+
+
+# Chunks in 1, 2, 8 and more than 8 spans of a trip with short last spans, and
+# the element counts around the folded kernels' change of cache policy
+# (2**26 bytes of state: 5592405 elements).
+@pytest.mark.parametrize("sizes,chunk", [((5000, 3, 2049), 2048), ((9000, 4097, 1), 4096), ((70_000, 16_385), 16384),
+                                         ((300_001, 65_537), 65536), ((2_592_405, 3_000_000), 4096),
+                                         ((2_592_406, 3_000_000), 4096)])
+@pytest.mark.parametrize("dtype", ["float16", None])
+@pytest.mark.parametrize("form", ["ragged", "flat"])
+def test_folded_steps_match_three_launches(gpu, sizes, chunk, dtype, form):
+    import torch
+    from distributedspeed_amd import _lib
+    from distributedspeed_amd.optimizers import AdamWOptimizer, MultiTensorAdamWOptimizer
+    _say(f"folded {form} {sizes} chunk={chunk} {dtype}")
+    dt = getattr(torch, dtype) if dtype else None
+    gen = torch.Generator(device=gpu).manual_seed(len(sizes))
+    init = [torch.empty(k, device=gpu).normal_(0.0, 0.02, generator=gen) for k in sizes]
+    grads = [torch.empty(k, device=gpu).normal_(0.0, 1e-3, generator=gen).to(dt or torch.float32) for k in sizes]
+
+    def steps(bound):
+        ps = [torch.nn.Parameter(t.clone()) for t in init]
+        kw = {"chunk_elems": chunk} if form == "ragged" else {}
+        cls = MultiTensorAdamWOptimizer if form == "ragged" else AdamWOptimizer
+        opt = cls(ps, lr=1e-3, param_dtype=dt, device=gpu, max_grad_norm=1.0, **kw)
+        _lib.call("dsx_set_tuning_fold", bound)
+        try:
+            for _ in range(3):
+                for p, g in zip(ps, grads):
+                    p.grad = g.clone()
+                opt.step()
+            torch.cuda.synchronize()
+        finally:
+            _lib.call("dsx_set_tuning_fold", 3 << 23)
+        return ps, opt
+
+    (pa, a), (pb, b) = steps(3 << 23), steps(0)
+    assert bytes(a.read_state()) == bytes(b.read_state())
+    for x, y in zip(pa, pb):
+        assert _bits(x.data, y.data)
+        for key in ("master", "exp_avg", "exp_avg_sq"):
+            assert _bits(a.state[x][key], b.state[y][key]), key
