@@ -835,6 +835,22 @@ __global__ __launch_bounds__(64) void k_store_groups(DsxGroupsDev g, DsxGroupsDe
   for (int i = threadIdx.x; i < (int)(sizeof(DsxGroupsDev) / 8); i += 64) out[i] = src[i];
 }
 
+// The grad pointers of `count` tensor records from `first` on, passed by value
+// as k_store_groups' block is: one small launch in stream order, where a
+// copy of the table from pinned memory took a pinned allocation, a DMA
+// submission and, of the host, about 15 us more a step.
+template <int N>
+struct GradPtrs {
+  const void* g[N];
+};
+
+template <int N>
+__global__ __launch_bounds__(N) void k_set_grads(GradPtrs<N> a, int32_t first, int32_t count,
+                                                 DsxTensorRef* __restrict__ tensors) {
+  const int i = threadIdx.x;
+  if (i < count) tensors[first + i].grad = a.g[i];
+}
+
 __global__ void k_state_init(DsxState* state, float scale, int32_t hysteresis) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     DsxState s = {};
@@ -1993,6 +2009,16 @@ int zero_step_flat(float* master, float* m, float* v, void* p16, int pdt, const 
   return rc;
 }
 
+template <int N>
+void launch_set_grads(DsxTensorRef* tensors, const void* const* grads, int32_t n, hipStream_t s) {
+  for (int32_t a = 0; a < n; a += N) {
+    GradPtrs<N> p = {};
+    const int32_t count = n - a < N ? n - a : N;
+    memcpy(p.g, grads + a, sizeof(void*) * (size_t)count);
+    hipLaunchKernelGGL(k_set_grads<N>, dim3(1), dim3(N), 0, s, p, a, count, tensors);
+  }
+}
+
 // The address of `scratch` on the current device, resolved once per device
 // with hipGetSymbolAddress (each GPU holds its own copy at its own address)
 // and checked to be the device the stream runs on.
@@ -2618,6 +2644,13 @@ int dsx_reduce_segments(const double* partials, const int64_t* offsets, int32_t 
   hipLaunchKernelGGL(k_reduce_segments, dim3((unsigned)nseg), dim3(kBlock), 0, as_stream(stream), partials, offsets,
                      out);
   return launch_status("dsx_reduce_segments");
+}
+
+int dsx_set_grads(DsxTensorRef* tensors, const void* const* grads, int32_t ntensors, void* stream) {
+  if (ntensors < 0 || (ntensors > 0 && (!tensors || !grads))) return fail(DSX_EINVAL, "bad tensor table or grads");
+  if (ntensors <= 64) launch_set_grads<64>(tensors, grads, ntensors, as_stream(stream));
+  else launch_set_grads<256>(tensors, grads, ntensors, as_stream(stream));
+  return launch_status("dsx_set_grads");
 }
 
 int dsx_unscale_norm_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks, int grad_dtype,

@@ -482,7 +482,7 @@ class ChunkTable:
         # them before update_grads points the table at the new ones.
         self._held = (list(masters), list(exp_avgs), list(exp_avg_sqs),
                       list(params16) if params16 is not None else None)
-        self._refs = refs
+        self._numels = list(numels)
         self._gdtype = grads[0].dtype
         self.tensors = torch.frombuffer(bytearray(bytes(refs)), dtype=torch.uint8).to(dev)
         self.chunks = torch.frombuffer(bytearray(bytes(chunks)), dtype=torch.uint8).to(dev)
@@ -490,18 +490,20 @@ class ChunkTable:
     def update_grads(self, grads) -> None:
         """Point the tensor table at new grad tensors (same count, numels and
         dtype) in place: the chunk table and every launch bound to this table
-        stay valid. The new table is copied from pinned memory on the current
-        stream, so launches already queued read the old one and later ones the
-        new one."""
-        refs = self._refs
-        if len(grads) != len(refs):
-            raise ValueError(f"expected {len(refs)} grads, got {len(grads)}")
+        stay valid. The pointers travel with a small launch on the current
+        stream, so launches already queued read the old ones and later ones the
+        new ones."""
+        if len(grads) != len(self._numels):
+            raise ValueError(f"expected {len(self._numels)} grads, got {len(grads)}")
         esz = torch.empty(0, dtype=self._gdtype).element_size()
         for i, g in enumerate(grads):
-            _need(g, f"grad[{i}]", self._gdtype, refs[i].numel, self.device, esz)
-            refs[i].grad = g.data_ptr()
-        host = torch.frombuffer(bytearray(bytes(refs)), dtype=torch.uint8).pin_memory()
-        self.tensors.copy_(host, non_blocking=True)
+            _need(g, f"grad[{i}]", self._gdtype, self._numels[i], self.device, esz)
+        self.set_grad_ptrs([g.data_ptr() for g in grads])
+
+    def set_grad_ptrs(self, ptrs) -> None:
+        """update_grads with addresses of grads that were checked already."""
+        k = len(self._numels)
+        _lib.call("dsx_set_grads", self.tensors.data_ptr(), (ctypes.c_void_p * k)(*ptrs), k, stream_of(self.device))
 
 
 def plan_unscale_norm_multi(table: ChunkTable, state: torch.Tensor, partials: torch.Tensor, nparts: int) -> Launch:

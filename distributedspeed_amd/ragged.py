@@ -118,7 +118,9 @@ class RaggedParams:
         self._own_chunks = bool(chunk_elems)
         self.ngroups = len(groups)
         self._table = None
-        self._key = None
+        self._grad_size = torch.empty(0, dtype=self.grad_dtype).element_size()
+        self._large = [m.numel() >= K2_TENSOR_ELEMS for m in self.master]
+        self._key = None  # the params' and the grads' addresses that the table holds
         self.k2_tensors: list[int] = []  # tensors the step runs through K2 (decided with each table)
         self.small_table = None  # K3's own table over the other tensors, where it has one
 
@@ -126,14 +128,14 @@ class RaggedParams:
         """Give every param a contiguous grad of the grad dtype on the device
         (zeros where autograd produced none, as the flat form does), 16-byte
         aligned for the tensors of K2's size (K2 takes them one by one)."""
-        for p in self.params:
+        dtype, device = self.grad_dtype, self.device
+        for p, large in zip(self.params, self._large):
             g = p.grad
             if g is None:
-                p.grad = torch.zeros_like(p, dtype=self.grad_dtype)
-            elif g.dtype != self.grad_dtype or g.device != self.device or not g.is_contiguous():
-                p.grad = g.to(self.device, self.grad_dtype).contiguous()
-        for p, m in zip(self.params, self.master):
-            if m.numel() >= K2_TENSOR_ELEMS and p.grad.data_ptr() % 16:
+                p.grad = torch.zeros_like(p, dtype=dtype)
+            elif g.dtype != dtype or g.device != device or not g.is_contiguous():
+                p.grad = g.to(device, dtype).contiguous()
+            if large and p.grad.data_ptr() % 16:
                 p.grad = p.grad.clone()  # a fresh allocation is aligned
 
     def table(self) -> ops.ChunkTable:
@@ -142,14 +144,18 @@ class RaggedParams:
         after zero_grad(set_to_none=True)), only the tensor table's grad
         pointers are refreshed, in place."""
         self.ensure_grads()
-        key = tuple((p.data_ptr(), p.grad.data_ptr()) for p in self.params)
-        if (self._table is not None and key != self._key
-                and all(a[0] == b[0] for a, b in zip(key, self._key))):
-            self._table.update_grads([p.grad for p in self.params])
-            if self.small_table is not None:
-                self.small_table.update_grads([self.params[i].grad for i in self._small])
-            self._key = key
-        if key != self._key:
+        homes = tuple([p.data_ptr() for p in self.params])
+        grads = tuple([p.grad.data_ptr() for p in self.params])
+        if self._table is not None and homes == self._key[0]:
+            if grads != self._key[1]:
+                size = self._grad_size
+                if any(p.grad.numel() != m.numel() or a % size for p, m, a in zip(self.params, self.master, grads)):
+                    raise ValueError("a grad's size or alignment does not match its parameter's")
+                self._table.set_grad_ptrs(grads)
+                if self.small_table is not None:
+                    self.small_table.set_grad_ptrs([grads[i] for i in self._small])
+                self._key = (homes, grads)
+        else:
             for p, m in zip(self.params, self.master):
                 if p.data.shape != m.shape or (self.param_dtype is None and p.data.data_ptr() != m.data_ptr()):
                     raise RuntimeError("a parameter's storage was replaced after the optimizer was built")
@@ -159,7 +165,7 @@ class RaggedParams:
             self._table = ops.ChunkTable(self.master, self.exp_avg, self.exp_avg_sq, p16,
                                          [p.grad for p in self.params], self.group_of, self.chunk_elems)
             self._split(p16)
-            self._key = key
+            self._key = (homes, grads)
         return self._table
 
     def _split(self, p16) -> None:

@@ -498,6 +498,13 @@ int dsx_zero_step_flat_noalloc(float* master, float* exp_avg,
 
 /* ---- K3: ragged lists (multi-tensor apply) ---------------------------- */
 
+/* Points a device tensor table's records at new grads, in stream order:
+ * tensors[i].grad = grads[i] for i < ntensors (grads is a host array, read
+ * before the call returns). For lists whose grads autograd allocates anew at
+ * every iteration; the chunk table stays. No counterpart in the reference. */
+int dsx_set_grads(DsxTensorRef* tensors, const void* const* grads,
+                  int32_t ntensors, void* stream);
+
 /* K1 over the chunks of a tensor list (tensors/chunks are device arrays).
  * Replaces the per-tensor loop of Src/zero/utils.py:147-152. */
 int dsx_unscale_norm_multi(const DsxTensorRef* tensors, const DsxChunk* chunks,

@@ -124,3 +124,41 @@ def test_folded_steps_match_three_launches(gpu, sizes, chunk, dtype, form):
         assert _bits(x.data, y.data)
         for key in ("master", "exp_avg", "exp_avg_sq"):
             assert _bits(a.state[x][key], b.state[y][key]), key
+
+
+@pytest.mark.parametrize("k", [1, 64, 65, 256, 257, 700])  # the launches' edges: 64 and 256 pointers
+def test_set_grads_points_every_record_at_its_grad(gpu, k):
+    import torch
+    from distributedspeed_amd import ops
+    from distributedspeed_amd._lib import DsxTensorRef
+    _say(f"set_grads k={k}")
+    ms = [torch.zeros(8, device=gpu) for _ in range(k)]
+    old = [torch.zeros(8, device=gpu) for _ in range(k)]
+    new = [torch.full((8,), float(i), device=gpu) for i in range(k)]
+    table = ops.ChunkTable(ms, ms, ms, None, old, chunk_elems=8)
+    before = table.tensors.cpu().numpy().tobytes()
+    table.update_grads(new)
+    torch.cuda.synchronize()
+    after = table.tensors.cpu().numpy().tobytes()
+    want = bytearray()
+    size = len(before) // k
+    for i in range(k):
+        ref = DsxTensorRef.from_buffer_copy(before, i * size)
+        ref.grad = new[i].data_ptr()
+        want += bytes(ref)
+    assert after == bytes(want)
+    with pytest.raises(ValueError):
+        table.update_grads(new[:-1] + [torch.zeros(9, device=gpu)])
+
+
+def test_a_grad_of_another_size_is_refused(gpu):
+    import torch
+    from distributedspeed_amd.optimizers import MultiTensorAdamWOptimizer
+    p = torch.nn.Parameter(torch.zeros(64, device=gpu))
+    opt = MultiTensorAdamWOptimizer([p], param_dtype=torch.bfloat16, device=gpu)
+    p.grad = torch.ones(64, device=gpu, dtype=torch.bfloat16)
+    opt.step()
+    p.data = p.data[:32]  # the same address, half the elements
+    p.grad = torch.ones(32, device=gpu, dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        opt.step()
