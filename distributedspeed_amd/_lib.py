@@ -100,6 +100,10 @@ SIGNATURES = {
     "dsx_norm_partials": (_c.c_int, [_P, _c.c_int, _c.c_int64, _P, _c.c_double, _P, _c.c_int32, _P]),
     "dsx_norm_partials_multi": (_c.c_int, [_P, _P, _c.c_int64, _c.c_int, _P, _c.c_double, _P, _c.c_int32, _P]),
     "dsx_clip_prepare": (_c.c_int, [_P, _c.c_int32, _c.c_double, _c.c_double, _c.c_double, _P, _P, _P]),
+    "dsx_clip_grad_norm": (_c.c_int, [_P, _c.c_int, _c.c_int64, _c.c_double, _c.c_double, _c.c_double, _P, _c.c_int32,
+                                      _P, _P, _P]),
+    "dsx_clip_grad_norm_multi": (_c.c_int, [_P, _P, _c.c_int64, _c.c_int, _c.c_double, _c.c_double, _c.c_double, _P,
+                                            _c.c_int32, _P, _P, _P]),
     "dsx_finalize": (_c.c_int, [_P, _c.c_int32, _P, DsxScalerConfig, DsxAdamwHyper, _P, _c.c_int32, _P, _P]),
     "dsx_finalize_groups": (_c.c_int, [_P, _c.c_int32, _P, DsxScalerConfig, _P, _P, _P, _c.c_int32, _c.c_int32,
                                        _P, _P]),

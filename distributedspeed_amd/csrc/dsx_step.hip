@@ -353,9 +353,14 @@ __device__ __forceinline__ double block_sum(double x) {
 // ---- norms other than L2 (clip_grad_norm_'s norm_type) -----------------------
 // kNormSq: sum of x^2 (the L2 norm's square, as K1); kNormAbs: sum of |x|
 // (p = 1); kNormMax: max |x|, NaN if any x is NaN (p = inf, as
-// tensor.abs().max()); kNormPow: sum of |x|^p in fp64 (any other p > 0).
+// tensor.abs().max()); kNormInt: sum of |x|^p for p = 3 to 8, each power as a
+// product in fp64 (its first factor, the square of an fp32 value, is exact, so
+// p - 2 roundings, and none more than pow's at p = 3); kNormPow: sum of |x|^p in
+// fp64 through pow (any other p > 0), whose math the pass waits for: 1.0e8 bf16
+// elements 541 us through pow, as products 46 (p = 3), 58 (4) and 107 (8), p = 2
+// 30.
 // x is the unscaled fp32 grad; every accumulation is in fp64.
-enum NormKind { kNormSq = 0, kNormAbs = 1, kNormMax = 2, kNormPow = 3 };
+enum NormKind { kNormSq = 0, kNormAbs = 1, kNormMax = 2, kNormPow = 3, kNormInt = 4 };
 
 // Commutative on what it combines (sums, or maxima of magnitudes: no -0).
 template <int K>
@@ -369,7 +374,12 @@ __device__ __forceinline__ double norm_acc(double acc, float x, double p) {
   if constexpr (K == kNormSq) return __builtin_fma((double)x, (double)x, acc);
   else if constexpr (K == kNormAbs) return acc + fabs((double)x);
   else if constexpr (K == kNormMax) return norm_comb<K>(acc, fabs((double)x));
-  else return acc + pow(fabs((double)x), p);
+  else if constexpr (K == kNormInt) {
+    const double a = fabs((double)x);
+    double r = a * a;
+    for (int k = 2; k < (int)p; ++k) r *= a;
+    return acc + r;
+  } else return acc + pow(fabs((double)x), p);
 }
 
 // The elements of one 16-byte slot (8 16-bit grads or 4 fp32 grads).
@@ -561,17 +571,19 @@ __global__ __launch_bounds__(kBlock) void k1_norm_multi(const DsxTensorRef* __re
 template <int K>
 __global__ __launch_bounds__(kBlock) void k_clip_prepare(const double* __restrict__ partials, int32_t nparts,
                                                          double p, double max_norm, double clip_eps,
-                                                         DsxState* __restrict__ state, double* __restrict__ norm_out) {
+                                                         DsxState* __restrict__ state, double* __restrict__ norm_out,
+                                                         float* __restrict__ norm_out32) {
   double x = 0.0;
   for (int i = threadIdx.x; i < nparts; i += kBlock) x = norm_comb<K>(x, partials[i]);
   const double total = block_reduce<K>(x);
   if (threadIdx.x != 0) return;
   double norm = total;
   if constexpr (K == kNormSq) norm = sqrt(total);
-  else if constexpr (K == kNormPow) norm = pow(total, 1.0 / p);
+  else if constexpr (K == kNormPow || K == kNormInt) norm = pow(total, 1.0 / p);
   float coef = 1.0f;
   if (norm > max_norm) coef = (float)(max_norm / (norm + clip_eps));
-  *norm_out = norm;
+  if (norm_out != nullptr) *norm_out = norm;
+  if (norm_out32 != nullptr) *norm_out32 = (float)norm;
   state->clip_once_coef = coef;
   state->clip_once = 1;
 }
@@ -1931,7 +1943,11 @@ void launch_k3(int pd, int unroll, bool drain, dim3 grid, const DsxTensorRef* t,
 
 int norm_kind(double p, int* kind) {
   if (!(p > 0.0)) return fail(DSX_EINVAL, "norm_type must be > 0 (finite or inf), got %g", p);
-  *kind = __builtin_isinf(p) ? kNormMax : p == 2.0 ? kNormSq : p == 1.0 ? kNormAbs : kNormPow;
+  *kind = __builtin_isinf(p) ? kNormMax
+          : p == 2.0         ? kNormSq
+          : p == 1.0         ? kNormAbs
+          : p >= 3.0 && p <= 8.0 && p == floor(p) ? kNormInt
+                                                  : kNormPow;
   return DSX_OK;
 }
 
@@ -1952,6 +1968,7 @@ void launch_norm(int kind, bool multi, const void* g, int64_t n, const DsxTensor
     case kNormSq: launch_norm_k<GD, kNormSq>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
     case kNormAbs: launch_norm_k<GD, kNormAbs>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
     case kNormMax: launch_norm_k<GD, kNormMax>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
+    case kNormInt: launch_norm_k<GD, kNormInt>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
     default: launch_norm_k<GD, kNormPow>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
   }
 }
@@ -1964,6 +1981,30 @@ int do_norm(int gdt, int kind, bool multi, const void* g, int64_t n, const DsxTe
     default: launch_norm<DSX_F32>(kind, multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
   }
   return launch_status(multi ? "dsx_norm_partials_multi" : "dsx_norm_partials");
+}
+
+int check_clip(double max_norm, double clip_eps, const DsxState* state, const void* norm_out) {
+  if (!(max_norm >= 0.0)) return fail(DSX_EINVAL, "max_norm must be >= 0, got %g", max_norm);
+  if (!(clip_eps >= 0.0)) return fail(DSX_EINVAL, "Invalid clip_eps: %g", clip_eps);
+  if (!state || !norm_out) return fail(DSX_EINVAL, "null state or norm_out");
+  return DSX_OK;
+}
+
+// The norm into whichever of the two outputs is given.
+int do_clip_prepare(int kind, const double* partials, int32_t nparts, double norm_type, double max_norm,
+                    double clip_eps, DsxState* state, double* norm_out, float* norm_out32, hipStream_t s) {
+#define DSX_PREPARE(K)                                                                                          \
+  hipLaunchKernelGGL(k_clip_prepare<K>, dim3(1), dim3(kBlock), 0, s, partials, nparts, norm_type, max_norm, clip_eps, \
+                     state, norm_out, norm_out32)
+  switch (kind) {
+    case kNormSq: DSX_PREPARE(kNormSq); break;
+    case kNormAbs: DSX_PREPARE(kNormAbs); break;
+    case kNormMax: DSX_PREPARE(kNormMax); break;
+    case kNormInt: DSX_PREPARE(kNormInt); break;
+    default: DSX_PREPARE(kNormPow); break;
+  }
+#undef DSX_PREPARE
+  return launch_status("dsx_clip_prepare");
 }
 
 // Argument checks of the flat step, shared by dsx_zero_step_flat and its
@@ -2410,31 +2451,35 @@ int dsx_clip_prepare(const double* partials, int32_t nparts, double norm_type, d
   int kind = 0;
   int rc = norm_kind(norm_type, &kind);
   if (!rc) rc = check_parts(partials, nparts);
+  if (!rc) rc = check_clip(max_norm, clip_eps, state, norm_out);
   if (rc) return rc;
-  if (!(max_norm >= 0.0)) return fail(DSX_EINVAL, "max_norm must be >= 0, got %g", max_norm);
-  if (!(clip_eps >= 0.0)) return fail(DSX_EINVAL, "Invalid clip_eps: %g", clip_eps);
-  if (!state || !norm_out) return fail(DSX_EINVAL, "null state or norm_out");
-  hipStream_t s = as_stream(stream);
-  const dim3 grid(1), blk(kBlock);
-  switch (kind) {
-    case kNormSq:
-      hipLaunchKernelGGL(k_clip_prepare<kNormSq>, grid, blk, 0, s, partials, nparts, norm_type, max_norm, clip_eps,
-                         state, norm_out);
-      break;
-    case kNormAbs:
-      hipLaunchKernelGGL(k_clip_prepare<kNormAbs>, grid, blk, 0, s, partials, nparts, norm_type, max_norm, clip_eps,
-                         state, norm_out);
-      break;
-    case kNormMax:
-      hipLaunchKernelGGL(k_clip_prepare<kNormMax>, grid, blk, 0, s, partials, nparts, norm_type, max_norm, clip_eps,
-                         state, norm_out);
-      break;
-    default:
-      hipLaunchKernelGGL(k_clip_prepare<kNormPow>, grid, blk, 0, s, partials, nparts, norm_type, max_norm, clip_eps,
-                         state, norm_out);
-      break;
-  }
-  return launch_status("dsx_clip_prepare");
+  return do_clip_prepare(kind, partials, nparts, norm_type, max_norm, clip_eps, state, norm_out, nullptr,
+                         as_stream(stream));
+}
+
+int dsx_clip_grad_norm(const void* grad, int grad_dtype, int64_t n, double norm_type, double max_norm,
+                       double clip_eps, double* partials, int32_t nparts, DsxState* state, float* norm_out,
+                       void* stream) {
+  int rc = check_clip(max_norm, clip_eps, state, norm_out);
+  if (!rc) rc = dsx_norm_partials(grad, grad_dtype, n, state, norm_type, partials, nparts, stream);
+  if (rc) return rc;
+  int kind = 0;
+  norm_kind(norm_type, &kind);
+  return do_clip_prepare(kind, partials, nparts, norm_type, max_norm, clip_eps, state, nullptr, norm_out,
+                         as_stream(stream));
+}
+
+int dsx_clip_grad_norm_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks, int grad_dtype,
+                             double norm_type, double max_norm, double clip_eps, double* partials, int32_t nparts,
+                             DsxState* state, float* norm_out, void* stream) {
+  int rc = check_clip(max_norm, clip_eps, state, norm_out);
+  if (!rc)
+    rc = dsx_norm_partials_multi(tensors, chunks, nchunks, grad_dtype, state, norm_type, partials, nparts, stream);
+  if (rc) return rc;
+  int kind = 0;
+  norm_kind(norm_type, &kind);
+  return do_clip_prepare(kind, partials, nparts, norm_type, max_norm, clip_eps, state, nullptr, norm_out,
+                         as_stream(stream));
 }
 
 int dsx_finalize(const double* partials, int32_t nparts, DsxState* state, DsxScalerConfig scaler,

@@ -288,14 +288,14 @@ class _FusedAdamWBase(torch.optim.Optimizer):
         max_norm = float(max_norm)
         if not max_norm >= 0:
             raise ValueError(f"max_norm must be >= 0, got {max_norm}")
-        s = ops.stream_of(self.device)
-        self._norm_launch(p)(s)
-        if getattr(self, "_clip_norm", None) is None:
-            self._clip_norm = torch.zeros(1, dtype=torch.float64, device=self.device)
-        ops.clip_prepare(self.partials, self.nparts, p, max_norm, self.clip_eps, self.dstate, self._clip_norm)
-        return self._clip_norm[0].to(torch.float32)
+        out = torch.empty((), dtype=torch.float32, device=self.device)
+        name, grads = self._clip_call()
+        _lib.call(name, *grads, p, max_norm, self.clip_eps, self.partials.data_ptr(), self.nparts,
+                  self.dstate.data_ptr(), out.data_ptr(), ops.stream_of(self.device))
+        return out
 
-    def _norm_launch(self, p: float) -> ops.Launch:
+    def _clip_call(self) -> tuple[str, tuple]:
+        """The entry point for this storage form and its grad arguments."""
         raise NotImplementedError
 
     # ---- device-side values, read on demand --------------------------------------------------
@@ -603,9 +603,10 @@ class AdamWOptimizer(_FusedAdamWBase):
         self.flat.check_grads_bound()
         self._k1(ops.stream_of(self.device))
 
-    def _norm_launch(self, p: float) -> ops.Launch:
+    def _clip_call(self) -> tuple[str, tuple]:
         self.flat.check_grads_bound()
-        return ops.plan_norm_partials(self.flat.grad, self.dstate, p, self.partials, self.nparts)
+        g = self.flat.grad
+        return "dsx_clip_grad_norm", (g.data_ptr(), ops.grad_code(g.dtype), g.numel())
 
     def step_fused(self) -> None:
         """K1 -> K0 -> K2 on the current stream; no host synchronisation."""
@@ -740,9 +741,10 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
         k1, _ = self._plans()
         k1(ops.stream_of(self.device))
 
-    def _norm_launch(self, p: float) -> ops.Launch:
+    def _clip_call(self) -> tuple[str, tuple]:
         self._plans()
-        return ops.plan_norm_partials_multi(self.store.table(), self.dstate, p, self.partials, self.nparts)
+        t = self._plans_for
+        return "dsx_clip_grad_norm_multi", (t.tensors.data_ptr(), t.chunks.data_ptr(), t.nchunks, t.gdt)
 
     def step_fused(self) -> None:
         """K1 (list) -> K0 -> K3 on the current stream (with K2 for each large

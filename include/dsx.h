@@ -323,6 +323,21 @@ int dsx_clip_prepare(const double* partials, int32_t nparts, double norm_type,
                      double max_norm, double clip_eps, DsxState* state,
                      double* norm_out, void* stream);
 
+/* clip_grad_norm_ in one call: dsx_norm_partials (or _multi) and
+ * dsx_clip_prepare with the norm into *norm_out as fp32 (device), two
+ * launches. Src/zero/optimizer.py:324-341, Src/zero/utils.py:187-216. */
+int dsx_clip_grad_norm(const void* grad, int grad_dtype, int64_t n,
+                       double norm_type, double max_norm, double clip_eps,
+                       double* partials, int32_t nparts, DsxState* state,
+                       float* norm_out, void* stream);
+
+int dsx_clip_grad_norm_multi(const DsxTensorRef* tensors,
+                             const DsxChunk* chunks, int64_t nchunks,
+                             int grad_dtype, double norm_type,
+                             double max_norm, double clip_eps,
+                             double* partials, int32_t nparts, DsxState* state,
+                             float* norm_out, void* stream);
+
 /* ---- K0: finalize ------------------------------------------------------ */
 
 /* Reduce the partials; decide skip (non-finite sum); on a clean step advance
