@@ -7,6 +7,14 @@ The flags that matter for correctness:
                       where torch's kernels round (explicit fmaf only)
   -Xclang -target-feature -Xclang -packed-fp32-ops
                       no packed fp32 instructions (v_pk_*_f32)
+and for speed:
+  -mllvm -amdgpu-kernarg-preload-count=16
+                      a kernel's leading arguments (the buffers and sizes) are
+                      in scalar registers when its waves start, instead of
+                      being the first trip to memory of each: flat steps on
+                      MI355X 9.5 -> 9.2 us at 9.0e5 elements, 12.9 -> 12.6 at
+                      1.9e6, 18.5 -> 18.0 at 3.0e6, nothing from 7.1e6 on (8,
+                      14 and 16 registers alike)
 HIP's defaults keep fp32 division and sqrt correctly rounded and fp32
 denormals intact, which the element math relies on.
 """
@@ -34,6 +42,7 @@ def hipcc() -> str:
 def command(out: str = OUT, extra: list[str] | None = None) -> list[str]:
     return [hipcc(), f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
             "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+            "-mllvm", "-amdgpu-kernarg-preload-count=16",
             "-Wall", "-Wno-unused-function",
             f"-I{INCLUDE}", SRC, "-o", out] + list(extra or [])
 
