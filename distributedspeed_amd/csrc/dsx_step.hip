@@ -485,18 +485,20 @@ __device__ __forceinline__ double norm_chunk(const u4* g16, int64_t nvec, bool k
 // blocks read those two fields, which nothing else writes during the step,
 // while one of them writes the state's updated fields.
 
+__device__ __forceinline__ void begin_fold(DsxState* s) {
+  const int32_t armed = s->clip_once != 0 ? 1 : 0;
+  s->step_scale = s->scale;
+  s->step_t2 = 2 * s->t + armed;
+  s->clip_once = 0;
+}
+
 template <int GD, int U>
 __global__ __launch_bounds__(kBlock) void k1_unscale_norm(const void* __restrict__ gv, int64_t n,
                                                           const DsxState* state, double* __restrict__ partials,
                                                           DsxState* fold, int64_t keep) {
   using G = Grad<GD>;
   const float inv = inv_of(state->scale);
-  if (fold != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-    const int32_t armed = fold->clip_once != 0 ? 1 : 0;
-    fold->step_scale = fold->scale;
-    fold->step_t2 = 2 * fold->t + armed;
-    fold->clip_once = 0;
-  }
+  if (fold != nullptr && blockIdx.x == 0 && threadIdx.x == 0) begin_fold(fold);
   const u4* g16 = static_cast<const u4*>(gv);
   const typename G::elem* g = static_cast<const typename G::elem*>(gv);
   const int64_t nvec = n / G::per16;
@@ -640,9 +642,13 @@ __global__ __launch_bounds__(kBlock) void k1_copy_unscale_norm(const void* __res
 // out[b] = sum of partials[offsets[b] .. offsets[b + 1]), by block b, each
 // thread over a fixed stride and the block reduce in a fixed tree: the same
 // bits for the same partials.
+// fold != NULL: block 0 starts a folded step, as k1_unscale_norm does (a training
+// iteration of the 784-1024-1024-10 MLP 432 -> 410 us, K0 a launch of its own and
+// three calls from Python against one).
 __global__ __launch_bounds__(kBlock) void k_reduce_segments(const double* __restrict__ partials,
                                                             const int64_t* __restrict__ offsets,
-                                                            double* __restrict__ out) {
+                                                            double* __restrict__ out, DsxState* fold) {
+  if (fold != nullptr && blockIdx.x == 0 && threadIdx.x == 0) begin_fold(fold);
   const int64_t lo = offsets[blockIdx.x], hi = offsets[blockIdx.x + 1];
   double acc = 0.0;
   for (int64_t i = lo + threadIdx.x; i < hi; i += kBlock) acc += partials[i];
@@ -1289,12 +1295,7 @@ __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorR
   constexpr int kWaves = kBlock / 64;
   constexpr int kLanes = WAVE ? 64 : kBlock;
   const float inv = inv_of(state->scale);
-  if (fold != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {  // as k1_unscale_norm
-    const int32_t armed = fold->clip_once != 0 ? 1 : 0;
-    fold->step_scale = fold->scale;
-    fold->step_t2 = 2 * fold->t + armed;
-    fold->clip_once = 0;
-  }
+  if (fold != nullptr && blockIdx.x == 0 && threadIdx.x == 0) begin_fold(fold);
   double acc = 0.0;
   int64_t seen = 0;  // elements this block (or wave) has read
   const int lane = WAVE ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
@@ -2230,12 +2231,35 @@ int check_plan(const DsxFlatPlan& P) {
   return DSX_OK;
 }
 
+// A host group block for a plan of ngroups groups.
+int check_groups(const DsxGroupsDev& G, int32_t ngroups) {
+  if (G.ngroups != ngroups)
+    return fail(DSX_EINVAL, "the group block holds %d groups, the plan %d", G.ngroups, ngroups);
+  if (G.bc_len < 0) return fail(DSX_EINVAL, "bad bias-correction table length");
+  for (int k = 0; k < ngroups; ++k) {
+    const int rc = check_hyper(G.hyper[k]);
+    if (rc) return rc;
+    if (G.bc_len > 0 && !G.bc_table[k]) return fail(DSX_EINVAL, "null bias-correction table for group %d", k);
+    if (G.t_offset[k] < 0) return fail(DSX_EINVAL, "negative t_offset for group %d", k);
+  }
+  return DSX_OK;
+}
+
 // The step of a checked plan: two launches (K1, then each nonempty group's K2
 // with the finalize folded in, the first of them writing the state) where
 // the fold applies, else three (K1, K0, each nonempty group's K2). The group
 // block is the host's G (a kernel argument) or, when G is NULL, the block at
 // the device address Gdev (read by the kernels: the graph form).
-int plan_launches(const DsxFlatPlan& P, const DsxGroupsDev* G, const DsxGroupsDev* Gdev, hipStream_t s) {
+// With `seg`, the norm's partials were taken as the grads were copied in, and
+// the step's partials (P.partials, one per segment) come from them in place of
+// K1's pass.
+struct Segments {
+  const double* partials;
+  const int64_t* offsets;
+};
+
+int plan_launches(const DsxFlatPlan& P, const DsxGroupsDev* G, const DsxGroupsDev* Gdev, hipStream_t s,
+                  const Segments* seg = nullptr) {
   bool fold = fold_applies(P.n, P.nparts);
   bool first = !fold && fold_first_applies(P.n, P.nparts);  // fold K0 into the first part alone
   int64_t prev = 0;
@@ -2244,8 +2268,15 @@ int plan_launches(const DsxFlatPlan& P, const DsxGroupsDev* G, const DsxGroupsDe
     prev = P.group_end[k];
     if (len > 0 && len < 4) fold = first = false;  // the folded K2 takes at least one 4-element slot
   }
-  int rc = do_unscale_norm(P.grad, P.grad_dtype, P.n, P.state, P.partials, P.nparts, s,
-                           fold || first ? P.state : nullptr);
+  DsxState* const begin = fold || first ? P.state : nullptr;
+  int rc = DSX_OK;
+  if (seg) {
+    hipLaunchKernelGGL(k_reduce_segments, dim3((unsigned)P.nparts), dim3(kBlock), 0, s, seg->partials, seg->offsets,
+                       P.partials, begin);
+    rc = launch_status("dsx_zero_step_segments (reduce)");
+  } else {
+    rc = do_unscale_norm(P.grad, P.grad_dtype, P.n, P.state, P.partials, P.nparts, s, begin);
+  }
   if (!rc && !fold && !first) {
     if (G) {
       rc = do_finalize(P.partials, P.nparts, P.state, P.scaler, *G, P.out, s);
@@ -2605,20 +2636,24 @@ int dsx_zero_step_flat(float* master, float* exp_avg, float* exp_avg_sq, void* p
 
 int dsx_zero_step_plan(const DsxFlatPlan* plan, const DsxGroupsDev* groups, void* stream) {
   if (!plan || !groups) return fail(DSX_EINVAL, "null plan or groups");
-  const DsxFlatPlan& P = *plan;
-  const DsxGroupsDev& G = *groups;
-  int rc = check_plan(P);
+  int rc = check_plan(*plan);
+  if (!rc) rc = check_groups(*groups, plan->ngroups);
   if (rc) return rc;
-  if (G.ngroups != P.ngroups)
-    return fail(DSX_EINVAL, "the group block holds %d groups, the plan %d", G.ngroups, P.ngroups);
-  if (G.bc_len < 0) return fail(DSX_EINVAL, "bad bias-correction table length");
-  for (int k = 0; k < P.ngroups; ++k) {
-    rc = check_hyper(G.hyper[k]);
-    if (rc) return rc;
-    if (G.bc_len > 0 && !G.bc_table[k]) return fail(DSX_EINVAL, "null bias-correction table for group %d", k);
-    if (G.t_offset[k] < 0) return fail(DSX_EINVAL, "negative t_offset for group %d", k);
-  }
-  return plan_launches(P, &G, nullptr, as_stream(stream));
+  return plan_launches(*plan, groups, nullptr, as_stream(stream));
+}
+
+int dsx_zero_step_segments(const DsxFlatPlan* plan, const DsxGroupsDev* groups, const double* block_partials,
+                           const int64_t* offsets, double* partials, int32_t nseg, void* stream) {
+  if (!plan || !groups) return fail(DSX_EINVAL, "null plan or groups");
+  if (!block_partials || !offsets) return fail(DSX_EINVAL, "null block partials or offsets");
+  DsxFlatPlan P = *plan;
+  P.partials = partials;
+  P.nparts = nseg;
+  int rc = check_plan(P);
+  if (!rc) rc = check_groups(*groups, P.ngroups);
+  if (rc) return rc;
+  const Segments seg{block_partials, offsets};
+  return plan_launches(P, groups, nullptr, as_stream(stream), &seg);
 }
 
 int dsx_zero_step_dev(const DsxFlatPlan* plan, const DsxGroupsDev* groups_dev, void* stream) {
@@ -2687,7 +2722,7 @@ int dsx_reduce_segments(const double* partials, const int64_t* offsets, int32_t 
     return fail(DSX_EINVAL, "nseg must be in [1, %d] (got %d)", DSX_MAX_PARTIALS, nseg);
   if (!partials || !offsets || !out) return fail(DSX_EINVAL, "null partials, offsets or out");
   hipLaunchKernelGGL(k_reduce_segments, dim3((unsigned)nseg), dim3(kBlock), 0, as_stream(stream), partials, offsets,
-                     out);
+                     out, static_cast<DsxState*>(nullptr));
   return launch_status("dsx_reduce_segments");
 }
 

@@ -251,9 +251,10 @@ class FlatPartition:
         """From now on the hooks copy grads with dsx_copy_unscale_norm, which
         also writes the norm's fp64 block partials (a segment per parameter,
         unscaled by the loss scale in `state`, a DsxState). hook_norm_ready()
-        says when they describe the flat buffer exactly; reduce_hook_norm()
-        then sums each segment into hook_norm_partials (one per parameter),
-        from which K0 finalizes without a K1 pass. False (and off) for more
+        says when they describe the flat buffer exactly; the step (in one call,
+        or through reduce_hook_norm()) then sums each segment into
+        hook_norm_partials (one per parameter) and finalizes from those without
+        a K1 pass. False (and off) for more
         parameters than K0 reads."""
         from . import _lib, ops
         if not self.params or len(self.params) > _lib.DSX_MAX_PARTIALS:
@@ -306,6 +307,11 @@ class FlatPartition:
         in-place write touched the buffer afterwards (its version counter)."""
         return (self._hn_on and self._hn_armed and all(self._hn_fired)
                 and self.grad._version == self._hn_version)
+
+    def hook_norm_args(self) -> tuple:
+        """The segments as dsx_zero_step_segments takes them."""
+        return (self._hn_block.data_ptr(), self._hn_offsets.data_ptr(), self.hook_norm_partials.data_ptr(),
+                len(self.params))
 
     def reduce_hook_norm(self, stream) -> None:
         """hook_norm_partials[i] <- sum of parameter i's block partials (one

@@ -554,16 +554,22 @@ class AdamWOptimizer(_FusedAdamWBase):
         self._plan_fn = _lib.load().dsx_zero_step_plan
         self._plan_args = (ctypes.byref(P), ctypes.byref(self._gblock))
 
-    def _step_plan(self) -> None:
+    def _step_plan(self, hooked: bool) -> None:
         """K1 -> K0 -> K2 (or K1 and K2 with K0 folded in) through
-        dsx_zero_step_plan. The group block is refilled only when it must be
-        (_refresh_group_block); the scaler settings only when they changed."""
+        dsx_zero_step_plan, or with the norm from the hooks' copies in place of
+        K1 (hooked) through dsx_zero_step_segments. The group block is refilled
+        only when it must be (_refresh_group_block); the scaler settings only
+        when they changed."""
         self._refresh_group_block()
         sc = self.scaler
         skey = (sc.mode, sc.window, sc.hysteresis, sc.min_scale, sc.growth_factor, sc.backoff_factor)
         if skey != self._skey:
             self._plan.scaler = sc.to_c()
             self._skey = skey
+        if hooked:
+            _lib.call("dsx_zero_step_segments", *self._plan_args, *self.flat.hook_norm_args(),
+                      ops.stream_of(self.device))
+            return
         rc = self._plan_fn(*self._plan_args, ops.stream_of(self.device))
         if rc:
             raise _lib.DsxError("dsx_zero_step_plan", rc, _lib.last_error())
@@ -616,11 +622,12 @@ class AdamWOptimizer(_FusedAdamWBase):
             return
         self.flat.check_grads_bound()
         self.steps_issued += 1
-        if (self._plan is not None and self._skip_host is None
-                and not (self._k0_hook is not None and self.flat.hook_norm_ready())):
+        # whether the hooks' copies already took the norm's partials: no K1 pass
+        hooked = self._k0_hook is not None and self.flat.hook_norm_ready()
+        if self._plan is not None and self._skip_host is None:
             # one C call; with track_skips on, the three launches are issued
             # one by one so that the skip flag's copy sits between K0 and K2
-            self._step_plan()
+            self._step_plan(hooked)
             self.flat.disarm_hook_norm()
             return
         hs, tables, bc_len = self._hypers()
@@ -634,8 +641,7 @@ class AdamWOptimizer(_FusedAdamWBase):
             self._after_finalize()  # after the replay: waits for the graph's K2 too
             return
         s = ops.stream_of(self.device)
-        if self._k0_hook is not None and self.flat.hook_norm_ready():
-            # the hooks' copies already took the norm's partials: no K1 pass
+        if hooked:
             self.flat.reduce_hook_norm(s)
             self._k0_hook(self.scaler.to_c(), hs, tables, self._t_offsets, bc_len, s)
         else:

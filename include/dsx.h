@@ -476,6 +476,17 @@ typedef struct DsxFlatPlan {
 int dsx_zero_step_plan(const DsxFlatPlan* plan /* host */,
                        const DsxGroupsDev* groups /* host */, void* stream);
 
+/* dsx_zero_step_plan for grads that were copied in by dsx_copy_unscale_norm:
+ * the norm comes from its block partials (block_partials[offsets[b] ..
+ * offsets[b + 1]) of segment b, device) in place of K1's pass, through one
+ * partial per segment in partials[nseg] (device scratch, instead of the
+ * plan's): as dsx_reduce_segments, dsx_finalize_groups and dsx_adamw_flat per
+ * group, with the finalize folded in as dsx_zero_step_plan folds it. */
+int dsx_zero_step_segments(const DsxFlatPlan* plan, const DsxGroupsDev* groups,
+                           const double* block_partials,
+                           const int64_t* offsets, double* partials,
+                           int32_t nseg, void* stream);
+
 /* dsx_zero_step_plan with the group block in DEVICE memory (written, e.g.,
  * by dsx_groups_upload), read by the kernels when they run: the launches
  * can be recorded into a HIP graph once and replayed, with a new block
