@@ -1825,10 +1825,10 @@ void launch_k2_fold_pol(dim3 grid, float* p, float* m, float* v, uint16_t* o, co
 template <int GD, int PD>
 void launch_k2_fold(float* p, float* m, float* v, void* p16, const void* g, int64_t n, const double* partials,
                     int32_t nparts, DsxState* state, const DsxScalerConfig& scfg, const FoldGroups& fg,
-                    int group, bool writer, DsxStepScalars* out, hipStream_t s, int64_t blocks_per_cu, int pol) {
+                    int group, bool writer, DsxStepScalars* out, hipStream_t s, int pol) {
   const int64_t slots = n >> 2;
   int64_t blocks = ceil_div(slots > 0 ? slots : 1, (int64_t)kBlock * 2);
-  const int64_t cap = (int64_t)cu_count() * blocks_per_cu;
+  const int64_t cap = (int64_t)cu_count() * kK2OneTripPerCu;
   if (blocks > cap) blocks = cap;
   if (writer) blocks += 1;  // the block that writes the records and the state
   uint16_t* o = static_cast<uint16_t*>(p16);
@@ -1849,31 +1849,41 @@ template <int GD>
 void k2_fold_by_param(int pd, float* p, float* m, float* v, void* p16, const void* g, int64_t n,
                       const double* partials, int32_t nparts, DsxState* state, const DsxScalerConfig& scfg,
                       const FoldGroups& fg, int group, bool writer, DsxStepScalars* out, hipStream_t s,
-                      int64_t bpc, int pol) {
+                      int pol) {
   if (pd == DSX_BF16)
-    launch_k2_fold<GD, DSX_BF16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, bpc, pol);
+    launch_k2_fold<GD, DSX_BF16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, pol);
   else
-    launch_k2_fold<GD, DSX_F16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, bpc, pol);
+    launch_k2_fold<GD, DSX_F16>(p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s, pol);
 }
 
 bool fold_applies(int64_t n, int32_t nparts) {
   return g_tune.fold_max_elems > 0 && n >= 4 && n <= g_tune.fold_max_elems && nparts <= kFoldMaxParts;
 }
 
-// Above the fold's bound, K0 is folded into the first of K2's parts alone,
-// launched one block per CU (so that few blocks pay the partials' reduction),
-// and the other parts read the records that launch's writer block wrote.
+// Above the fold's bound, K0 is folded into a first part alone (k2_first_part),
+// and K2 over the rest reads the records that launch's writer block wrote.
 // Like the whole fold, it needs n >= 4 (a bound of 1 to 3 set through
 // dsx_set_tuning_fold would otherwise send 2 or 3 elements to it).
 bool fold_first_applies(int64_t n, int32_t nparts) {
   return g_tune.fold_max_elems > 0 && n >= 4 && n > g_tune.fold_max_elems && nparts <= kFoldMaxParts;
 }
 
-// The length of K2's first part over n elements (k2_dispatch's split).
+// The length of the part that K0 is folded into when a step above the fold's
+// bound folds it into its first part alone: what K2's one-trip grid covers, or
+// K2's own first part if that is shorter. In that grid the partials' reduction
+// and the decision cost the first trip's latency once; over a whole part of up
+// to 2^26 elements at one block per CU they came before a loop that is slower
+// than K2's. Flat steps, us, that / 2^20 / 2^22 / 2^24 elements / K0 as a launch:
+// 2.6e7 bf16 elements 129.2 / 129.5 / 129.9 / 127.8 / 129.6, 3.0e7 fp32 150.2 /
+// 151.4 / 152.0 / 146.1 / 151.6, 6.4e7 bf16 306.1 / 304.8 / 305.0 / 303.4 / 305.2,
+// 1.24e8 586.0 / 584.1 / 584.0 / 582.6 / 584.2, 1.0e9 4924 / 4916 / 4953 / 4911 /
+// 4920.
+constexpr int64_t kFoldFirstElems = int64_t(1) << 24;
 int64_t k2_first_part(int64_t n) {
   const int64_t want = g_tune.k2_chunk_elems;
-  if (want <= 0 || n <= want) return n;
-  return ceil_div(ceil_div(n, ceil_div(n, want)), 1024) * 1024;
+  int64_t part = n;
+  if (want > 0 && n > want) part = ceil_div(ceil_div(n, ceil_div(n, want)), 1024) * 1024;
+  return part < kFoldFirstElems ? part : kFoldFirstElems;
 }
 
 // The folded kernels' policy for a step over n elements.
@@ -1883,27 +1893,27 @@ int fold_policy(int nontemporal, int64_t n) {
   return n <= kKeepStateBytes / 12 ? kFoldKeep : kFoldSmall;
 }
 
-// The folded K2 over n elements: K2's one-trip grid (at most
-// kK2OneTripPerCu blocks per CU), or at most bpc blocks per CU. step_elems: the
-// elements of the whole step, by which the policy is chosen.
+// The folded K2 over n elements in K2's one-trip grid (at most kK2OneTripPerCu
+// blocks per CU). step_elems: the elements of the whole step, by which the
+// policy is chosen.
 int do_adamw_fold(float* p, float* m, float* v, void* p16, int pdt, const void* g, int gdt, int64_t n,
                   const double* partials, int32_t nparts, DsxState* state, const DsxScalerConfig& scfg,
                   const FoldGroups& fg, int group, bool writer, DsxStepScalars* out, hipStream_t s,
-                  int64_t step_elems, int64_t bpc = kK2OneTripPerCu) {
+                  int64_t step_elems) {
   const int pd = p16 ? pdt : DSX_F16;
   const int pol = fold_policy(g_tune.nontemporal, step_elems);
   switch (gdt) {
     case DSX_BF16:
       k2_fold_by_param<DSX_BF16>(pd, p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s,
-                                 bpc, pol);
+                                 pol);
       break;
     case DSX_F16:
       k2_fold_by_param<DSX_F16>(pd, p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s,
-                                 bpc, pol);
+                                 pol);
       break;
     default:
       k2_fold_by_param<DSX_F32>(pd, p, m, v, p16, g, n, partials, nparts, state, scfg, fg, group, writer, out, s,
-                                 bpc, pol);
+                                 pol);
       break;
   }
   return launch_status("dsx_adamw_flat (finalize folded in)");
@@ -2037,7 +2047,7 @@ int zero_step_flat(float* master, float* m, float* v, void* p16, int pdt, const 
     const int64_t a = k2_first_part(n);
     int rc = do_unscale_norm(g, gdt, n, state, partials, nparts, s, state);
     if (!rc) rc = do_adamw_fold(master, m, v, p16, pdt, g, gdt, a, partials, nparts, state, scaler,
-                                FoldGroups{&grp, nullptr, 1}, 0, true, out, s, n, 1);
+                                FoldGroups{&grp, nullptr, 1}, 0, true, out, s, n);
     if (!rc && a < n) {
       void* p16a = p16 ? static_cast<void*>(static_cast<uint16_t*>(p16) + a) : nullptr;
       const void* ga = static_cast<const char*>(g) + a * (gdt == DSX_F32 ? 4 : 2);
@@ -2304,7 +2314,7 @@ int plan_launches(const DsxFlatPlan& P, const DsxGroupsDev* G, const DsxGroupsDe
       // this group and the other groups read them.
       const int64_t c = k2_first_part(b - a);
       rc = do_adamw_fold(P.master + a, P.exp_avg + a, P.exp_avg_sq + a, p16, P.param_dtype, ga, P.grad_dtype, c,
-                         P.partials, P.nparts, P.state, P.scaler, fg, k, true, P.out, s, P.n, 1);
+                         P.partials, P.nparts, P.state, P.scaler, fg, k, true, P.out, s, P.n);
       if (!rc && c < b - a) {
         void* p16c = p16 ? static_cast<void*>(static_cast<uint16_t*>(p16) + c) : nullptr;
         rc = do_adamw_flat(P.master + a + c, P.exp_avg + a + c, P.exp_avg_sq + a + c, p16c, P.param_dtype,

@@ -223,7 +223,7 @@ int dsx_set_tuning_k2_chunk(int64_t chunk_elems);
  * state and the step records). The folded K2 takes K2's one-trip grid (2
  * slots per thread, at most 32 blocks per CU) whatever dsx_set_tuning and
  * dsx_set_tuning_k2 set. Above max_elems (same limits), K0's finalize is
- * folded into the first of K2's parts alone, launched one block per CU, and
+ * folded into the first of K2's parts alone, and
  * the other parts read the records it writes. 0 always runs K1, K0, K2.
  * Default 3 * 2^23 (one and a half sweeps of K2's one-trip grid on 256 CUs).
  * No counterpart in the reference. */
