@@ -2190,6 +2190,20 @@ int do_adamw_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t 
   return launch_status("dsx_adamw_multi");
 }
 
+// A chunk table over a tensor list; numel: the sum of its chunks' lengths, by
+// which only launch shapes are chosen.
+struct List {
+  const DsxTensorRef* tensors;
+  const DsxChunk* chunks;
+  int64_t nchunks, numel;
+};
+
+int check_list(const List& l) {
+  if (l.nchunks < 0 || (l.nchunks > 0 && (!l.tensors || !l.chunks))) return fail(DSX_EINVAL, "bad chunk table");
+  if (l.numel < 0) return fail(DSX_EINVAL, "numel must be >= 0");
+  return DSX_OK;
+}
+
 template <int GD, int PD>
 void launch_k3_fold_p(int pol, int32_t split, const DsxTensorRef* t, const DsxChunk* c, int64_t nc,
                       const double* partials, int32_t nparts, DsxState* state, const DsxScalerConfig& scfg,
@@ -2198,8 +2212,9 @@ void launch_k3_fold_p(int pol, int32_t split, const DsxTensorRef* t, const DsxCh
   hipLaunchKernelGGL((k3_adamw_fold<GD, PD, POL>), grid, dim3(kBlock), 0, s, t, c, nc, split, partials, nparts, state, \
                      scfg, grp, out)
   const dim3 grid((unsigned)(nc * split + 1));  // the chunks' spans, and the writer
-  switch (pol) {  // a list of the fold's size never streams
+  switch (pol) {
     case kFoldPlain: DSX_FOLD(kFoldPlain); break;
+    case kFoldStream: DSX_FOLD(kFoldStream); break;
     case kFoldSmall: DSX_FOLD(kFoldSmall); break;
     default: DSX_FOLD(kFoldKeep); break;
   }
@@ -2207,17 +2222,18 @@ void launch_k3_fold_p(int pol, int32_t split, const DsxTensorRef* t, const DsxCh
 }
 
 template <int GD>
-void launch_k3_fold(int pd, int64_t numel, const DsxTensorRef* t, const DsxChunk* c, int64_t nc, const double* partials,
-                    int32_t nparts, DsxState* state, const DsxScalerConfig& scfg, const DsxGroupsDev& grp,
-                    DsxStepScalars* out, hipStream_t s) {
+void launch_k3_fold(int pd, const List& l, int64_t step_elems, const double* partials, int32_t nparts, DsxState* state,
+                    const DsxScalerConfig& scfg, const DsxGroupsDev& grp, DsxStepScalars* out, hipStream_t s) {
   // Spans of one trip for chunks of the list's mean length, at most 8.
-  const int64_t trips = ceil_div(ceil_div(numel, nc), (int64_t)kBlock * 2 * 4);
+  const int64_t trips = ceil_div(ceil_div(l.numel, l.nchunks), (int64_t)kBlock * 2 * 4);
   const int32_t split = (int32_t)(trips < 1 ? 1 : trips > 8 ? 8 : trips);
-  const int pol = fold_policy(g_tune.k3_nontemporal, numel);
+  const int pol = fold_policy(g_tune.k3_nontemporal, step_elems);
   if (pd == DSX_BF16)
-    launch_k3_fold_p<GD, DSX_BF16>(pol, split, t, c, nc, partials, nparts, state, scfg, grp, out, s);
+    launch_k3_fold_p<GD, DSX_BF16>(pol, split, l.tensors, l.chunks, l.nchunks, partials, nparts, state, scfg, grp, out,
+                                   s);
   else
-    launch_k3_fold_p<GD, DSX_F16>(pol, split, t, c, nc, partials, nparts, state, scfg, grp, out, s);
+    launch_k3_fold_p<GD, DSX_F16>(pol, split, l.tensors, l.chunks, l.nchunks, partials, nparts, state, scfg, grp, out,
+                                  s);
 }
 
 // The flat plan's own checks (everything but the group block).
@@ -2253,6 +2269,88 @@ int check_groups(const DsxGroupsDev& G, int32_t ngroups) {
     if (G.t_offset[k] < 0) return fail(DSX_EINVAL, "negative t_offset for group %d", k);
   }
   return DSX_OK;
+}
+
+int do_k3_fold(const List& l, int64_t step_elems, int pdt, int gdt, const double* partials, int32_t nparts,
+               DsxState* state, const DsxScalerConfig& scaler, const DsxGroupsDev& G, DsxStepScalars* out,
+               hipStream_t s) {
+  switch (gdt) {
+    case DSX_BF16: launch_k3_fold<DSX_BF16>(pdt, l, step_elems, partials, nparts, state, scaler, G, out, s); break;
+    case DSX_F16: launch_k3_fold<DSX_F16>(pdt, l, step_elems, partials, nparts, state, scaler, G, out, s); break;
+    default: launch_k3_fold<DSX_F32>(pdt, l, step_elems, partials, nparts, state, scaler, G, out, s); break;
+  }
+  return launch_status("K3 (finalize folded in)");
+}
+
+// The step over a list: the norm over the table `norm`, the update of the
+// tensors of the host array k2 through K2 one by one and of the table `k3`
+// through K3. Two launches where the fold applies (3 * 2^23 elements are 24
+// chunks of 4096 per CU), one table serves both and has few chunks. Above
+// the fold's bound K0 is folded into a first part alone, as in the flat form:
+// K3's first chunks, about kFoldFirstElems elements, or the first K2 tensor's
+// first part (us a step against K0 as a launch of its own and the rest called
+// from Python one by one: 4.0e7 bf16 elements 222 -> 204, 8.0e7 414 -> 395, 1.5e8
+// 763 -> 735, 2.5e8 1275 -> 1233). Else K0 is a launch of its own.
+int list_step(const List& norm, const List& k3, const DsxTensorRef* k2, int32_t nk2, int64_t numel, int pdt, int gdt,
+              DsxState* state, const DsxScalerConfig& scaler, const DsxGroupsDev* groups, double* partials,
+              int32_t nparts, DsxStepScalars* out, hipStream_t s) {
+  if (!is_grad_dtype(gdt)) return fail(DSX_EINVAL, "grad dtype must be DSX_F16, DSX_BF16 or DSX_F32 (got %d)", gdt);
+  if (!is16(pdt)) return fail(DSX_EINVAL, "param16 dtype must be DSX_F16 or DSX_BF16 (got %d)", pdt);
+  int rc = check_list(norm);
+  if (!rc) rc = check_list(k3);
+  if (rc) return rc;
+  if (nk2 < 0 || (nk2 > 0 && !k2)) return fail(DSX_EINVAL, "bad K2 tensors");
+  if (!state || !out || !groups) return fail(DSX_EINVAL, "null state, scalars or groups");
+  rc = check_parts(partials, nparts);
+  if (!rc) rc = check_scaler(scaler);
+  if (rc) return rc;
+  const DsxGroupsDev& G = *groups;
+  if (G.ngroups < 1 || G.ngroups > DSX_MAX_GROUPS)
+    return fail(DSX_EINVAL, "ngroups must be in [1, %d] (got %d)", DSX_MAX_GROUPS, G.ngroups);
+  rc = check_groups(G, G.ngroups);
+  for (int32_t i = 0; !rc && i < nk2; ++i) {
+    rc = check_flat(k2[i].master, k2[i].exp_avg, k2[i].exp_avg_sq, k2[i].param16, pdt, k2[i].grad, gdt, k2[i].numel);
+    if (!rc && (k2[i].group < 0 || k2[i].group >= G.ngroups))
+      rc = fail(DSX_EINVAL, "K2 tensor %d is of group %d of %d", i, k2[i].group, G.ngroups);
+  }
+  if (rc) return rc;
+  const int64_t few = kK3FoldChunksPerCu * cu_count();
+  const bool whole = nk2 == 0 && k3.chunks == norm.chunks && k3.nchunks > 0 && fold_applies(numel, nparts) &&
+                     k3.nchunks <= few;
+  const bool first = !whole && fold_first_applies(numel, nparts) && (k3.nchunks > 0 || (nk2 > 0 && k2[0].numel >= 4));
+  rc = do_unscale_norm_multi(norm.tensors, norm.chunks, norm.nchunks, gdt, state, partials, nparts, s,
+                             whole || first ? state : nullptr);
+  if (!rc && !whole && !first) rc = do_finalize(partials, nparts, state, scaler, G, out, s);
+  int64_t chunks = 0, elems = 0;  // stepped by the folded launch: K3's chunks, or elements of the first K2 tensor
+  if (!rc && whole) {
+    chunks = k3.nchunks;
+  } else if (!rc && first && k3.nchunks > 0) {
+    chunks = kFoldFirstElems / (ceil_div(k3.numel, k3.nchunks) + 1);
+    if (chunks < 1) chunks = 1;
+    if (chunks > few) chunks = few;
+    if (chunks > k3.nchunks) chunks = k3.nchunks;
+  } else if (!rc && first) {
+    const DsxTensorRef& t = k2[0];
+    elems = k2_first_part(t.numel);
+    rc = do_adamw_fold(t.master, t.exp_avg, t.exp_avg_sq, t.param16, pdt, t.grad, gdt, elems, partials, nparts, state,
+                       scaler, FoldGroups{&G, nullptr, 1}, t.group, true, out, s, numel);
+  }
+  if (!rc && chunks > 0) {
+    const int64_t mean = ceil_div(k3.numel, k3.nchunks);
+    rc = do_k3_fold(List{k3.tensors, k3.chunks, chunks, chunks * (mean < kFoldFirstElems ? mean : kFoldFirstElems)},
+                    numel, pdt, gdt, partials, nparts, state, scaler, G, out, s);
+  }
+  const int64_t gsz = gdt == DSX_F32 ? 4 : 2;
+  for (int32_t i = 0; !rc && i < nk2; ++i) {
+    const DsxTensorRef& t = k2[i];
+    const int64_t a = i == 0 ? elems : 0;
+    void* p16 = t.param16 ? static_cast<void*>(static_cast<uint16_t*>(t.param16) + a) : nullptr;
+    rc = do_adamw_flat(t.master + a, t.exp_avg + a, t.exp_avg_sq + a, p16, pdt,
+                       static_cast<const char*>(t.grad) + a * gsz, gdt, t.numel - a, out + t.group, s);
+  }
+  if (!rc)
+    rc = do_adamw_multi(k3.tensors, k3.chunks + chunks, k3.nchunks - chunks, pdt, gdt, out, s);
+  return rc;
 }
 
 // The step of a checked plan: two launches (K1, then each nonempty group's K2
@@ -2769,46 +2867,19 @@ int dsx_zero_step_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int
                         int param_dtype, int grad_dtype, DsxState* state, DsxScalerConfig scaler,
                         const DsxGroupsDev* groups, double* partials, int32_t nparts, DsxStepScalars* out,
                         void* stream) {
-  if (!is_grad_dtype(grad_dtype))
-    return fail(DSX_EINVAL, "grad dtype must be DSX_F16, DSX_BF16 or DSX_F32 (got %d)", grad_dtype);
-  if (!is16(param_dtype)) return fail(DSX_EINVAL, "param16 dtype must be DSX_F16 or DSX_BF16 (got %d)", param_dtype);
-  if (nchunks < 0 || (nchunks > 0 && (!tensors || !chunks))) return fail(DSX_EINVAL, "bad chunk table");
-  if (numel < 0) return fail(DSX_EINVAL, "numel must be >= 0");
-  if (!state || !out || !groups) return fail(DSX_EINVAL, "null state, scalars or groups");
-  int rc = check_parts(partials, nparts);
-  if (!rc) rc = check_scaler(scaler);
-  if (rc) return rc;
-  const DsxGroupsDev& G = *groups;
-  if (G.ngroups < 1 || G.ngroups > DSX_MAX_GROUPS)
-    return fail(DSX_EINVAL, "ngroups must be in [1, %d] (got %d)", DSX_MAX_GROUPS, G.ngroups);
-  if (G.bc_len < 0) return fail(DSX_EINVAL, "bad bias-correction table length");
-  for (int k = 0; k < G.ngroups; ++k) {
-    rc = check_hyper(G.hyper[k]);
-    if (rc) return rc;
-    if (G.bc_len > 0 && !G.bc_table[k]) return fail(DSX_EINVAL, "null bias-correction table for group %d", k);
-    if (G.t_offset[k] < 0) return fail(DSX_EINVAL, "negative t_offset for group %d", k);
-  }
-  hipStream_t s = as_stream(stream);
-  // Two launches where the fold applies (3 * 2^23 elements are 24 chunks of
-  // 4096 per CU) and the list has few chunks; else K1, K0, K3.
-  const bool fold = nchunks > 0 && fold_applies(numel, nparts) && nchunks <= kK3FoldChunksPerCu * cu_count();
-  rc = do_unscale_norm_multi(tensors, chunks, nchunks, grad_dtype, state, partials, nparts, s,
-                             fold ? state : nullptr);
-  if (rc) return rc;
-  if (!fold) {
-    rc = do_finalize(partials, nparts, state, scaler, G, out, s);
-    if (!rc) rc = do_adamw_multi(tensors, chunks, nchunks, param_dtype, grad_dtype, out, s);
-    return rc;
-  }
-  switch (grad_dtype) {
-    case DSX_BF16: launch_k3_fold<DSX_BF16>(param_dtype, numel, tensors, chunks, nchunks, partials, nparts, state,
-                                            scaler, G, out, s); break;
-    case DSX_F16: launch_k3_fold<DSX_F16>(param_dtype, numel, tensors, chunks, nchunks, partials, nparts, state,
-                                          scaler, G, out, s); break;
-    default: launch_k3_fold<DSX_F32>(param_dtype, numel, tensors, chunks, nchunks, partials, nparts, state, scaler,
-                                     G, out, s); break;
-  }
-  return launch_status("dsx_zero_step_multi (finalize folded in)");
+  const List all{tensors, chunks, nchunks, numel};
+  return list_step(all, all, nullptr, 0, numel, param_dtype, grad_dtype, state, scaler, groups, partials, nparts, out,
+                   as_stream(stream));
+}
+
+int dsx_zero_step_lists(const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks, int64_t numel,
+                        const DsxTensorRef* k3_tensors, const DsxChunk* k3_chunks, int64_t k3_nchunks,
+                        int64_t k3_numel, const DsxTensorRef* k2_tensors, int32_t nk2, int param_dtype, int grad_dtype,
+                        DsxState* state, DsxScalerConfig scaler, const DsxGroupsDev* groups, double* partials,
+                        int32_t nparts, DsxStepScalars* out, void* stream) {
+  return list_step(List{tensors, chunks, nchunks, numel}, List{k3_tensors, k3_chunks, k3_nchunks, k3_numel}, k2_tensors,
+                   nk2, numel, param_dtype, grad_dtype, state, scaler, groups, partials, nparts, out,
+                   as_stream(stream));
 }
 
 }  // extern "C"

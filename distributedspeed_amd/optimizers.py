@@ -720,15 +720,27 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
                               st.master[i].numel(), base + ops.SCALARS_BYTES * st.group_of[i])
                              for i in st.k2_tensors]
             self._k2_meta = (pdt, gdt)
-            # The whole step in one call (dsx_zero_step_multi) when one table
-            # serves K1 and K3: its fixed arguments, bound once per table.
-            self._one_call = None
+            # The whole step in one call, its fixed arguments bound once per
+            # table: dsx_zero_step_multi when one table serves K1 and K3,
+            # dsx_zero_step_lists otherwise.
+            lib = _lib.load()
+            end = (ctypes.byref(self._gblock), ops._ptr(self.partials), int(self.nparts), ops._ptr(self.scalars))
+            head = (ops._ptr(table.tensors), ops._ptr(table.chunks), ctypes.c_int64(table.nchunks),
+                    ctypes.c_int64(table.numel))
+            self._k2_refs = None
             if k3_table is table:
-                self._one_call = (_lib.load().dsx_zero_step_multi,
-                                  (ops._ptr(table.tensors), ops._ptr(table.chunks), ctypes.c_int64(table.nchunks),
-                                   ctypes.c_int64(table.numel), table.pdt, table.gdt, ops._ptr(self.dstate)),
-                                  (ctypes.byref(self._gblock), ops._ptr(self.partials), int(self.nparts),
-                                   ops._ptr(self.scalars)))
+                self._one_call = ("dsx_zero_step_multi", lib.dsx_zero_step_multi,
+                                  head + (table.pdt, table.gdt, ops._ptr(self.dstate)), end)
+            else:
+                k3 = ((None, None, 0, 0) if k3_table is None else
+                      (ops._ptr(k3_table.tensors), ops._ptr(k3_table.chunks), k3_table.nchunks, k3_table.numel))
+                self._k2_refs = (_lib.DsxTensorRef * max(1, len(self._k2_each)))()
+                for ref, (p, mp, ep, vp, pp, n, _), i in zip(self._k2_refs, self._k2_each, st.k2_tensors):
+                    ref.master, ref.exp_avg, ref.exp_avg_sq, ref.param16 = mp, ep, vp, pp
+                    ref.grad, ref.numel, ref.group = p.grad.data_ptr(), n, st.group_of[i]
+                self._one_call = ("dsx_zero_step_lists", lib.dsx_zero_step_lists,
+                                  head + k3 + (self._k2_refs, len(self._k2_each), table.pdt, table.gdt,
+                                               ops._ptr(self.dstate)), end)
             self._plans_for = table
         return self._k1, self._k3
 
@@ -754,22 +766,24 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
 
     def step_fused(self) -> None:
         """K1 (list) -> K0 -> K3 on the current stream (with K2 for each large
-        tensor when the list is in K3's one-block-per-CU range); no host
-        synchronisation (a chunk-table rebuild, after storage moved, uploads
+        tensor of a mid-size list); no host synchronisation (a chunk-table rebuild, after storage moved, uploads
         the new table)."""
         self._note_stepped()
         k1, k3 = self._plans()
         self.steps_issued += 1
         s = ops.stream_of(self.device)
-        if self._one_call is not None and self._skip_host is None:
-            # one C call (K1, K0, K3, or K1 and K3 with K0 folded in); with
-            # track_skips on, the launches stay separate so that the skip
-            # flag's copy sits between K0 and K3
+        if self._skip_host is None:
+            # one C call (K1, K0, K2 and K3, with K0 folded in where it can
+            # be); with track_skips on, the launches stay separate so that the
+            # skip flag's copy sits between K0 and K3
             self._refresh_group_block()
-            fn, head, tail = self._one_call
+            name, fn, head, tail = self._one_call
+            if self._k2_refs is not None:
+                for ref, each in zip(self._k2_refs, self._k2_each):
+                    ref.grad = each[0].grad.data_ptr()
             rc = fn(*head, self.scaler.to_c(), *tail, s)
             if rc:
-                raise _lib.DsxError("dsx_zero_step_multi", rc, _lib.last_error())
+                raise _lib.DsxError(name, rc, _lib.last_error())
             return
         hs, tables, bc_len = self._hypers()
         k1(s)

@@ -223,8 +223,8 @@ int dsx_set_tuning_k2_chunk(int64_t chunk_elems);
  * state and the step records). The folded K2 takes K2's one-trip grid (2
  * slots per thread, at most 32 blocks per CU) whatever dsx_set_tuning and
  * dsx_set_tuning_k2 set. Above max_elems (same limits), K0's finalize is
- * folded into the first of K2's parts alone, and
- * the other parts read the records it writes. 0 always runs K1, K0, K2.
+ * folded into a first part of at most 2^24 elements alone, and K2 over the
+ * rest reads the records it writes. 0 always runs K1, K0, K2.
  * Default 3 * 2^23 (one and a half sweeps of K2's one-trip grid on 256 CUs).
  * No counterpart in the reference. */
 int dsx_set_tuning_fold(int64_t max_elems);
@@ -549,9 +549,10 @@ int dsx_adamw_multi(const DsxTensorRef* tensors, const DsxChunk* chunks,
  * HOST group block `groups` (as dsx_finalize_groups takes it; checked here),
  * K3 -- or, for lists of at most dsx_set_tuning_fold's bound in elements
  * (numel, the sum of the chunk lengths) with at most 512 partials and at
- * most 20 chunks per CU, two launches: K1 recording the entry values, and K3
+ * most 24 chunks per CU, two launches: K1 recording the entry values, and K3
  * with K0's finalize folded in (every block decides the step with K0's code;
- * one extra block writes the state and the records), the same bits. out
+ * one extra block writes the state and the records), the same bits; above
+ * that bound K0 is folded into K3's first chunks alone. out
  * holds groups->ngroups records. Replaces ZeROOptimizer.step over a list of
  * tensors (Src/zero/optimizer.py:212-274, torch AdamW's per-tensor loop
  * behind Src/zero/stage2.py:609-612). */
@@ -559,6 +560,21 @@ int dsx_zero_step_multi(const DsxTensorRef* tensors, const DsxChunk* chunks,
                         int64_t nchunks, int64_t numel, int param_dtype,
                         int grad_dtype, DsxState* state, DsxScalerConfig scaler,
                         const DsxGroupsDev* groups /* host */, double* partials,
+                        int32_t nparts, DsxStepScalars* out, void* stream);
+
+/* dsx_zero_step_multi with the update split: the norm over the whole list's
+ * chunk table (numel elements), K3 over a table of its own (k3_numel elements;
+ * k3_nchunks may be 0), and K2 over each tensor of the HOST array
+ * k2_tensors[nk2], whose arrays are 16-byte aligned. Each tensor of the list is
+ * in one of the two. */
+int dsx_zero_step_lists(const DsxTensorRef* tensors, const DsxChunk* chunks,
+                        int64_t nchunks, int64_t numel,
+                        const DsxTensorRef* k3_tensors,
+                        const DsxChunk* k3_chunks, int64_t k3_nchunks,
+                        int64_t k3_numel, const DsxTensorRef* k2_tensors,
+                        int32_t nk2, int param_dtype, int grad_dtype,
+                        DsxState* state, DsxScalerConfig scaler,
+                        const DsxGroupsDev* groups, double* partials,
                         int32_t nparts, DsxStepScalars* out, void* stream);
 
 #ifdef __cplusplus

@@ -162,3 +162,50 @@ def test_a_grad_of_another_size_is_refused(gpu):
     p.grad = torch.ones(32, device=gpu, dtype=torch.bfloat16)
     with pytest.raises(ValueError):
         opt.step()
+
+
+# Lists above the fold's bound: K0 folded into K3's first chunks (one table; its
+# own table; before K2's tensors) or into the first K2 tensor's first part,
+# against K0 as a launch of its own.
+@pytest.mark.parametrize("sizes,chunk", [((3000, 70_001, 5), 8), ((13_000_008, 9_000_001, 14_000_000), None),
+                                         ((77, 17_000_000, 20_000_000), None), ((18_000_000, 17_000_000), None)])
+def test_lists_fold_k0_into_a_first_part(gpu, sizes, chunk):
+    import torch
+    from distributedspeed_amd import _lib
+    from distributedspeed_amd.flat_step import ScalerConfig
+    from distributedspeed_amd.optimizers import MultiTensorAdamWOptimizer
+    _say(f"list fold {sizes}")
+    gen = torch.Generator(device=gpu).manual_seed(8)
+    init = [torch.empty(k, device=gpu).normal_(0.0, 0.02, generator=gen) for k in sizes]
+    grads = [torch.empty(k, device=gpu).normal_(0.0, 1.0, generator=gen).half() for k in sizes]
+
+    def steps(bound):
+        ps = [torch.nn.Parameter(t.clone()) for t in init]
+        gs = [{"params": ps[:1]}, {"params": ps[1:], "lr": 3e-4, "weight_decay": 0.0}]
+        opt = MultiTensorAdamWOptimizer(gs, lr=1e-3, param_dtype=torch.float16, device=gpu, max_grad_norm=1.0,
+                                        loss_scaler=ScalerConfig(mode="dynamic", init_scale=1024.0, hysteresis=1),
+                                        chunk_elems=chunk)
+        _lib.call("dsx_set_tuning_fold", bound)
+        try:
+            for step in range(4):
+                for p, g in zip(ps, grads):
+                    p.grad = g.clone()
+                if step == 1:
+                    ps[-1].grad[3] = float("inf")
+                if step == 2:
+                    opt.clip_grad_norm_(0.01)
+                opt.step()
+            torch.cuda.synchronize()
+        finally:
+            _lib.call("dsx_set_tuning_fold", 3 << 23)
+        return ps, opt
+
+    # a bound of 1000 elements sends the small list past it as well
+    (pa, a), (pb, b) = steps(1000 if chunk else 3 << 23), steps(0)
+    assert bytes(a.read_state()) == bytes(b.read_state()) and a.read_state().overflow_count == 1
+    for g in range(2):
+        assert bytes(a.last_scalars(g)) == bytes(b.last_scalars(g))
+    for x, y in zip(pa, pb):
+        assert _bits(x.data, y.data)
+        for key in ("master", "exp_avg", "exp_avg_sq"):
+            assert _bits(a.state[x][key], b.state[y][key]), key
