@@ -122,6 +122,8 @@ SIGNATURES = {
     "dsx_set_grads": (_c.c_int, [_P, _P, _c.c_int32, _P]),
     "dsx_unscale_norm_multi": (_c.c_int, [_P, _P, _c.c_int64, _c.c_int, _P, _P, _c.c_int32, _P]),
     "dsx_adamw_multi": (_c.c_int, [_P, _P, _c.c_int64, _c.c_int, _c.c_int, _P, _P]),
+    "dsx_zero_step_multi_moved": (_c.c_int, [_P, _P, _c.c_int64, _c.c_int64, _c.c_int, _c.c_int, _P, DsxScalerConfig,
+                                             _P, _P, _c.c_int32, _P, _P, _c.c_int32, _P]),
     "dsx_zero_step_lists": (_c.c_int, [_P, _P, _c.c_int64, _c.c_int64, _P, _P, _c.c_int64, _c.c_int64, _P, _c.c_int32,
                                        _c.c_int, _c.c_int, _P, DsxScalerConfig, _P, _P, _c.c_int32, _P, _P]),
     "dsx_zero_step_multi": (_c.c_int, [_P, _P, _c.c_int64, _c.c_int64, _c.c_int, _c.c_int, _P, DsxScalerConfig, _P,

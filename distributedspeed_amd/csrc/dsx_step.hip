@@ -843,6 +843,12 @@ __global__ __launch_bounds__(kBlock) void k0_finalize_dev(const double* __restri
   finalize_body(sumsq, state, scfg, grp, groups_bad_dev(grp, max_groups), max_groups, out);
 }
 
+// Grad pointers passed by value through the kernel-argument segment.
+template <int N>
+struct GradPtrs {
+  const void* g[N];
+};
+
 // Writes a group block passed by value (through the kernel-argument
 // segment, so no DMA copy and no host staging buffer) to device memory,
 // 8 bytes per lane.
@@ -857,11 +863,6 @@ __global__ __launch_bounds__(64) void k_store_groups(DsxGroupsDev g, DsxGroupsDe
 // as k_store_groups' block is: one small launch in stream order, where a
 // copy of the table from pinned memory took a pinned allocation, a DMA
 // submission and, of the host, about 15 us more a step.
-template <int N>
-struct GradPtrs {
-  const void* g[N];
-};
-
 template <int N>
 __global__ __launch_bounds__(N) void k_set_grads(GradPtrs<N> a, int32_t first, int32_t count,
                                                  DsxTensorRef* __restrict__ tensors) {
@@ -1284,18 +1285,25 @@ __device__ __forceinline__ Sc scalars_rec(const DsxStepScalars* scalars, int32_t
 // one trip of one wave). The next chunk's record is requested with the
 // current chunk's tensor record, so that it is in by the time the current
 // chunk is done.
-template <int GD, bool WAVE>
+//
+// NP > 1: the grads are at the addresses in gp, by tensor, and the last block
+// also stores those in the table's records, for the launches after this one (a
+// small list whose grads moved: one launch less than k_set_grads and K1, the
+// MLP's list 22.5 -> 18.3 us a step).
+template <int GD, bool WAVE, int NP>
 __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorRef* __restrict__ tensors,
                                                                 const DsxChunk* __restrict__ chunks,
                                                                 int64_t nchunks, const DsxState* state,
                                                                 double* __restrict__ partials, DsxState* fold,
-                                                                int64_t keep) {
+                                                                int64_t keep, DsxTensorRef* __restrict__ table,
+                                                                int32_t count, GradPtrs<NP> gp) {
   using G = Grad<GD>;
   constexpr int U = 4;
   constexpr int kWaves = kBlock / 64;
   constexpr int kLanes = WAVE ? 64 : kBlock;
   const float inv = inv_of(state->scale);
   if (fold != nullptr && blockIdx.x == 0 && threadIdx.x == 0) begin_fold(fold);
+  if (NP > 1 && blockIdx.x == gridDim.x - 1 && (int)threadIdx.x < count) table[threadIdx.x].grad = gp.g[threadIdx.x];
   double acc = 0.0;
   int64_t seen = 0;  // elements this block (or wave) has read
   const int lane = WAVE ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
@@ -1305,7 +1313,8 @@ __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorR
   if (c < nchunks) {  // the grid is the partial count, which may exceed the chunk count
     DsxChunk ch = chunk_rec(chunks, c);
     for (;;) {
-      const typename G::elem* g = static_cast<const typename G::elem*>(tensor_rec(tensors, ch.tensor).grad) + ch.start;
+      const void* base = NP > 1 ? gp.g[ch.tensor] : tensor_rec(tensors, ch.tensor).grad;
+      const typename G::elem* g = static_cast<const typename G::elem*>(base) + ch.start;
       const int64_t cn = c + stride;
       const DsxChunk chn = chunk_rec(chunks, cn < nchunks ? cn : c);
       int64_t done = 0;
@@ -2101,15 +2110,36 @@ int noalloc_scratch(hipStream_t s, unsigned char** out) {
   return DSX_OK;
 }
 
+// The addresses that a list's grads have moved to (count of them, at most
+// kMovedGrads), and the table whose records are to hold them.
+constexpr int kMovedGrads = 64;
+struct MovedGrads {
+  DsxTensorRef* table;
+  const void* const* grads;
+  int32_t count;
+};
+
+template <int GD, bool WAVE>
+void launch_k1_multi_w(dim3 grid, const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks,
+                       const DsxState* state, double* partials, DsxState* fold, const MovedGrads* moved,
+                       hipStream_t s) {
+  const int64_t keep = keep_elems(GD, (int64_t)grid.x * (WAVE ? kWaves : 1));
+  if (moved) {
+    GradPtrs<kMovedGrads> gp = {};
+    memcpy(gp.g, moved->grads, sizeof(void*) * (size_t)moved->count);
+    hipLaunchKernelGGL((k1_unscale_norm_multi<GD, WAVE, kMovedGrads>), grid, dim3(kBlock), 0, s, tensors, chunks,
+                       nchunks, state, partials, fold, keep, moved->table, moved->count, gp);
+  } else {
+    hipLaunchKernelGGL((k1_unscale_norm_multi<GD, WAVE, 1>), grid, dim3(kBlock), 0, s, tensors, chunks, nchunks, state,
+                       partials, fold, keep, static_cast<DsxTensorRef*>(nullptr), 0, GradPtrs<1>{});
+  }
+}
+
 template <int GD>
 void launch_k1_multi(bool wave, dim3 grid, const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks,
-                     const DsxState* state, double* partials, DsxState* fold, hipStream_t s) {
-  if (wave)
-    hipLaunchKernelGGL((k1_unscale_norm_multi<GD, true>), grid, dim3(kBlock), 0, s, tensors, chunks, nchunks,
-                       state, partials, fold, keep_elems(GD, (int64_t)grid.x * kWaves));
-  else
-    hipLaunchKernelGGL((k1_unscale_norm_multi<GD, false>), grid, dim3(kBlock), 0, s, tensors, chunks, nchunks,
-                       state, partials, fold, keep_elems(GD, grid.x));
+                     const DsxState* state, double* partials, DsxState* fold, const MovedGrads* moved, hipStream_t s) {
+  if (wave) launch_k1_multi_w<GD, true>(grid, tensors, chunks, nchunks, state, partials, fold, moved, s);
+  else launch_k1_multi_w<GD, false>(grid, tensors, chunks, nchunks, state, partials, fold, moved, s);
 }
 
 // K1 over a chunk table. Each wave takes its own chunks when the table has
@@ -2124,13 +2154,14 @@ void launch_k1_multi(bool wave, dim3 grid, const DsxTensorRef* tensors, const Ds
 // slower one wave per chunk.
 constexpr int64_t kK1WaveChunksPerPart = 16;
 int do_unscale_norm_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks, int gdt,
-                          const DsxState* state, double* partials, int32_t nparts, hipStream_t s, DsxState* fold) {
+                          const DsxState* state, double* partials, int32_t nparts, hipStream_t s, DsxState* fold,
+                          const MovedGrads* moved = nullptr) {
   const dim3 grid(nparts);
   const bool wave = nchunks <= kK1WaveChunksPerPart * nparts;
   switch (gdt) {
-    case DSX_BF16: launch_k1_multi<DSX_BF16>(wave, grid, tensors, chunks, nchunks, state, partials, fold, s); break;
-    case DSX_F16: launch_k1_multi<DSX_F16>(wave, grid, tensors, chunks, nchunks, state, partials, fold, s); break;
-    default: launch_k1_multi<DSX_F32>(wave, grid, tensors, chunks, nchunks, state, partials, fold, s); break;
+    case DSX_BF16: launch_k1_multi<DSX_BF16>(wave, grid, tensors, chunks, nchunks, state, partials, fold, moved, s); break;
+    case DSX_F16: launch_k1_multi<DSX_F16>(wave, grid, tensors, chunks, nchunks, state, partials, fold, moved, s); break;
+    default: launch_k1_multi<DSX_F32>(wave, grid, tensors, chunks, nchunks, state, partials, fold, moved, s); break;
   }
   return launch_status("dsx_unscale_norm_multi");
 }
@@ -2293,7 +2324,7 @@ int do_k3_fold(const List& l, int64_t step_elems, int pdt, int gdt, const double
 // 763 -> 735, 2.5e8 1275 -> 1233). Else K0 is a launch of its own.
 int list_step(const List& norm, const List& k3, const DsxTensorRef* k2, int32_t nk2, int64_t numel, int pdt, int gdt,
               DsxState* state, const DsxScalerConfig& scaler, const DsxGroupsDev* groups, double* partials,
-              int32_t nparts, DsxStepScalars* out, hipStream_t s) {
+              int32_t nparts, DsxStepScalars* out, hipStream_t s, const MovedGrads* moved = nullptr) {
   if (!is_grad_dtype(gdt)) return fail(DSX_EINVAL, "grad dtype must be DSX_F16, DSX_BF16 or DSX_F32 (got %d)", gdt);
   if (!is16(pdt)) return fail(DSX_EINVAL, "param16 dtype must be DSX_F16 or DSX_BF16 (got %d)", pdt);
   int rc = check_list(norm);
@@ -2319,7 +2350,7 @@ int list_step(const List& norm, const List& k3, const DsxTensorRef* k2, int32_t 
                      k3.nchunks <= few;
   const bool first = !whole && fold_first_applies(numel, nparts) && (k3.nchunks > 0 || (nk2 > 0 && k2[0].numel >= 4));
   rc = do_unscale_norm_multi(norm.tensors, norm.chunks, norm.nchunks, gdt, state, partials, nparts, s,
-                             whole || first ? state : nullptr);
+                             whole || first ? state : nullptr, moved);
   if (!rc && !whole && !first) rc = do_finalize(partials, nparts, state, scaler, G, out, s);
   int64_t chunks = 0, elems = 0;  // stepped by the folded launch: K3's chunks, or elements of the first K2 tensor
   if (!rc && whole) {
@@ -2870,6 +2901,19 @@ int dsx_zero_step_multi(const DsxTensorRef* tensors, const DsxChunk* chunks, int
   const List all{tensors, chunks, nchunks, numel};
   return list_step(all, all, nullptr, 0, numel, param_dtype, grad_dtype, state, scaler, groups, partials, nparts, out,
                    as_stream(stream));
+}
+
+int dsx_zero_step_multi_moved(DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks, int64_t numel,
+                              int param_dtype, int grad_dtype, DsxState* state, DsxScalerConfig scaler,
+                              const DsxGroupsDev* groups, double* partials, int32_t nparts, DsxStepScalars* out,
+                              const void* const* grads, int32_t ntensors, void* stream) {
+  if (ntensors < 1 || ntensors > kMovedGrads)
+    return fail(DSX_EINVAL, "ntensors must be in [1, %d] (got %d)", kMovedGrads, ntensors);
+  if (!tensors || !grads) return fail(DSX_EINVAL, "bad tensor table or grads");
+  const List all{tensors, chunks, nchunks, numel};
+  const MovedGrads moved{tensors, grads, ntensors};
+  return list_step(all, all, nullptr, 0, numel, param_dtype, grad_dtype, state, scaler, groups, partials, nparts, out,
+                   as_stream(stream), &moved);
 }
 
 int dsx_zero_step_lists(const DsxTensorRef* tensors, const DsxChunk* chunks, int64_t nchunks, int64_t numel,

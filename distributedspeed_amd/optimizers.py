@@ -702,8 +702,8 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
                 else:
                     p.grad.zero_()
 
-    def _plans(self):
-        table = self.store.table()
+    def _plans(self, carry: bool = False):
+        table = self.store.table(carry)
         if table is not self._plans_for:  # rebuilt after storage moved: bind again
             st = self.store
             self._k1 = ops.plan_unscale_norm_multi(table, self.dstate, self.partials, self.nparts)
@@ -728,6 +728,7 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
             head = (ops._ptr(table.tensors), ops._ptr(table.chunks), ctypes.c_int64(table.nchunks),
                     ctypes.c_int64(table.numel))
             self._k2_refs = None
+            self._moved_fn = lib.dsx_zero_step_multi_moved
             if k3_table is table:
                 self._one_call = ("dsx_zero_step_multi", lib.dsx_zero_step_multi,
                                   head + (table.pdt, table.gdt, ops._ptr(self.dstate)), end)
@@ -769,7 +770,7 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
         tensor of a mid-size list); no host synchronisation (a chunk-table rebuild, after storage moved, uploads
         the new table)."""
         self._note_stepped()
-        k1, k3 = self._plans()
+        k1, k3 = self._plans(carry=self._skip_host is None)
         self.steps_issued += 1
         s = ops.stream_of(self.device)
         if self._skip_host is None:
@@ -781,9 +782,16 @@ class MultiTensorAdamWOptimizer(_FusedAdamWBase):
             if self._k2_refs is not None:
                 for ref, each in zip(self._k2_refs, self._k2_each):
                     ref.grad = each[0].grad.data_ptr()
-            rc = fn(*head, self.scaler.to_c(), *tail, s)
+            moved = self.store.moved
+            if moved is None:
+                rc = fn(*head, self.scaler.to_c(), *tail, s)
+            else:  # the first launch carries the grads' new addresses
+                name = "dsx_zero_step_multi_moved"
+                rc = self._moved_fn(*head, self.scaler.to_c(), *tail, moved, len(moved), s)
             if rc:
                 raise _lib.DsxError(name, rc, _lib.last_error())
+            if moved is not None:
+                self.store.moved_set()
             return
         hs, tables, bc_len = self._hypers()
         k1(s)

@@ -18,6 +18,8 @@ param's or a grad's storage has moved (checked every step on the host).
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import ops
@@ -38,6 +40,7 @@ from . import ops
 K2_TENSOR_ELEMS = 1 << 24
 K3_SMALL_PER_CU = 20
 K3_MANY_PER_CU = 256
+MOVED_MAX = 64  # grad pointers that a step's first launch carries
 
 
 def auto_chunk_elems(numel: int) -> int:
@@ -120,6 +123,7 @@ class RaggedParams:
         self._table = None
         self._grad_size = torch.empty(0, dtype=self.grad_dtype).element_size()
         self._large = [m.numel() >= K2_TENSOR_ELEMS for m in self.master]
+        self.moved = None  # moved grads' addresses that a step is to carry to the table
         self._key = None  # the params' and the grads' addresses that the table holds
         self.k2_tensors: list[int] = []  # tensors the step runs through K2 (decided with each table)
         self.small_table = None  # K3's own table over the other tensors, where it has one
@@ -138,11 +142,14 @@ class RaggedParams:
             if large and p.grad.data_ptr() % 16:
                 p.grad = p.grad.clone()  # a fresh allocation is aligned
 
-    def table(self) -> ops.ChunkTable:
+    def table(self, carry: bool = False) -> ops.ChunkTable:
         """The device chunk table for the current storage: rebuilt when a
         param's address changed; when only grads moved (autograd's own grads
         after zero_grad(set_to_none=True)), only the tensor table's grad
-        pointers are refreshed, in place."""
+        pointers are refreshed, in place. With `carry`, a small list's are
+        left in self.moved for a launch that takes them along
+        (dsx_zero_step_multi_moved); the caller then reports moved_set()."""
+        self.moved = None
         self.ensure_grads()
         homes = tuple([p.data_ptr() for p in self.params])
         grads = tuple([p.grad.data_ptr() for p in self.params])
@@ -151,6 +158,10 @@ class RaggedParams:
                 size = self._grad_size
                 if any(p.grad.numel() != m.numel() or a % size for p, m, a in zip(self.params, self.master, grads)):
                     raise ValueError("a grad's size or alignment does not match its parameter's")
+                if carry and self.small_table is None and not self.k2_tensors and len(grads) <= MOVED_MAX:
+                    self.moved = (ctypes.c_void_p * len(grads))(*grads)
+                    self._moved_key = (homes, grads)
+                    return self._table
                 self._table.set_grad_ptrs(grads)
                 if self.small_table is not None:
                     self.small_table.set_grad_ptrs([grads[i] for i in self._small])
@@ -167,6 +178,10 @@ class RaggedParams:
             self._split(p16)
             self._key = (homes, grads)
         return self._table
+
+    def moved_set(self) -> None:
+        """The pointers in self.moved are in the table, in stream order."""
+        self._key, self.moved = self._moved_key, None
 
     def _split(self, p16) -> None:
         """Choose the tensors that step through K2 for the table just built,

@@ -562,6 +562,19 @@ int dsx_zero_step_multi(const DsxTensorRef* tensors, const DsxChunk* chunks,
                         const DsxGroupsDev* groups /* host */, double* partials,
                         int32_t nparts, DsxStepScalars* out, void* stream);
 
+/* dsx_zero_step_multi for a list whose grads have moved to the addresses in
+ * grads[ntensors] (a HOST array, read before the call returns; at most 64
+ * tensors, which is all of the list): as dsx_set_grads and then the step, with
+ * the addresses carried by the step's first launch. */
+int dsx_zero_step_multi_moved(DsxTensorRef* tensors, const DsxChunk* chunks,
+                              int64_t nchunks, int64_t numel, int param_dtype,
+                              int grad_dtype, DsxState* state,
+                              DsxScalerConfig scaler,
+                              const DsxGroupsDev* groups, double* partials,
+                              int32_t nparts, DsxStepScalars* out,
+                              const void* const* grads, int32_t ntensors,
+                              void* stream);
+
 /* dsx_zero_step_multi with the update split: the norm over the whole list's
  * chunk table (numel elements), K3 over a table of its own (k3_numel elements;
  * k3_nchunks may be 0), and K2 over each tensor of the HOST array

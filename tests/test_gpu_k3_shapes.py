@@ -209,3 +209,38 @@ def test_lists_fold_k0_into_a_first_part(gpu, sizes, chunk):
         assert _bits(x.data, y.data)
         for key in ("master", "exp_avg", "exp_avg_sq"):
             assert _bits(a.state[x][key], b.state[y][key]), key
+
+
+# Lists whose grads move at every step, at the most pointers that a step's
+# first launch carries and one more, with the norm asked for in between.
+@pytest.mark.parametrize("k", [1, 64, 65])
+@pytest.mark.parametrize("size", [40, 3000])
+def test_moving_grads_reach_every_launch(gpu, k, size):
+    import torch
+    from distributedspeed_amd.optimizers import AdamWOptimizer, MultiTensorAdamWOptimizer
+    _say(f"moving grads k={k} size={size}")
+    gen = torch.Generator(device=gpu).manual_seed(k)
+    init = [torch.empty(size + i % 5, device=gpu).normal_(0.0, 0.02, generator=gen) for i in range(k)]
+    opts = []
+    for cls in (AdamWOptimizer, MultiTensorAdamWOptimizer):
+        ps = [torch.nn.Parameter(t.clone()) for t in init]
+        opts.append((ps, cls(ps, lr=1e-3, param_dtype=torch.bfloat16, device=gpu)))
+    held = []  # every step's grads stay alive, so each step's are elsewhere
+    for step in range(6):
+        grads = [torch.empty(t.numel(), device=gpu).normal_(0.0, 1.0, generator=gen).bfloat16() for t in init]
+        held.append(grads)
+        for ps, opt in opts:
+            for p, g in zip(ps, grads):
+                p.grad = g if step % 2 else g.clone()
+            if step == 3:
+                opt.clip_grad_norm_(1e9)  # reads the grads, clips nothing
+            if step == 4:
+                opt.track_skips(True)
+            if step == 5:
+                opt.track_skips(False)
+            opt.step()
+    torch.cuda.synchronize()
+    for pf, pr in zip(opts[0][0], opts[1][0]):
+        assert _bits(pf.data, pr.data)
+        for key in ("master", "exp_avg", "exp_avg_sq"):
+            assert _bits(opts[0][1].state[pf][key], opts[1][1].state[pr][key]), key
