@@ -114,6 +114,18 @@ class HostStateStreamer:
         self.ev_out = [torch.cuda.Event() for _ in range(self.nbuf)]
         self.ev_step = torch.cuda.Event()  # the last run(), whatever stream it was on
         self.last_bytes = 0  # host<->HBM bytes the last run() moved (both directions)
+        self._held = ()  # the state that the last in-place run() steps
+
+    def __del__(self):
+        if getattr(self, "_held", ()):
+            self.ev_step.synchronize()  # the state may go with this streamer
+
+    @staticmethod
+    def _in_place(host_state) -> bool:
+        """Whether K2 can take the state where it is: pinned, fp32 and
+        contiguous with every array on a 16-byte boundary, as K2 reads it."""
+        return all(t.is_pinned() and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                   for t in host_state)
 
     @property
     def stage(self) -> list:
@@ -128,13 +140,19 @@ class HostStateStreamer:
             copy_only: bool = False) -> None:
         """pieces: (start, end, scalars) ranges of the flat partition, each
         with the DsxStepScalars (device uint8[64]) of its parameter group.
-        Pinned state is stepped in place; other host memory is staged.
+        Pinned state is stepped in place; host memory that a kernel cannot
+        touch, or K2 cannot read (_in_place), is staged.
         copy_only (measurement only): the staged copies, streams and events
         with the AdamW launch left out, so every chunk goes back unchanged;
         param16, grad and the scalars are then unused."""
         compute = torch.cuda.current_stream(self.device)
         compute.wait_event(self.ev_step)
-        if not copy_only and all(t.is_pinned() for t in host_state):
+        if not copy_only and self._in_place(host_state):
+            # A kernel's use of pinned memory is not known to torch's pinned
+            # allocator as a copy's is, so the arrays are kept until it is over.
+            if self._held and any(x is not y for x, y in zip(self._held, host_state)):
+                self.ev_step.synchronize()
+            self._held = tuple(host_state)
             for a, b, scal in pieces:
                 ops.adamw_host_state(*(t[a:b] for t in host_state),
                                      param16[a:b] if param16 is not None else None, grad[a:b], scal)

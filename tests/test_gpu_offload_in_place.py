@@ -96,3 +96,22 @@ def test_the_streamer_takes_pinned_and_pageable_state(gpu, pinned):
     for name, h, t in zip(("master", "exp_avg", "exp_avg_sq"), host, (p, m, v)):
         assert _bits(h, t), name
     assert _bits(o16, p16)
+
+
+def test_pinned_state_off_k2s_alignment_is_staged(gpu):
+    """Views that start 4 bytes into a pinned array: K2 reads 16 bytes at a
+    time, so they take the staged path, as all pinned state once did."""
+    import torch
+    from distributedspeed_amd.offload import HostStateStreamer
+    n = 9_001
+    p, m, v, p16, g = _inputs(n, torch.bfloat16, torch.bfloat16, gpu, 5)
+    host = [_pinned(torch.cat([t[:1], t]))[1:] for t in (p, m, v)]
+    o16 = p16.clone()
+    st = HostStateStreamer(gpu, 4096)
+    st.run(tuple(host), o16, g, [(0, n, _scalars(gpu))])
+    from distributedspeed_amd import ops
+    ops.adamw_flat(p, m, v, p16, g, _scalars(gpu))
+    torch.cuda.synchronize()
+    for name, h, t in zip(("master", "exp_avg", "exp_avg_sq"), host, (p, m, v)):
+        assert _bits(h, t), name
+    assert _bits(o16, p16)
