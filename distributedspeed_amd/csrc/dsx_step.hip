@@ -353,12 +353,11 @@ __device__ __forceinline__ double block_sum(double x) {
 // ---- norms other than L2 (clip_grad_norm_'s norm_type) -----------------------
 // kNormSq: sum of x^2 (the L2 norm's square, as K1); kNormAbs: sum of |x|
 // (p = 1); kNormMax: max |x|, NaN if any x is NaN (p = inf, as
-// tensor.abs().max()); kNormInt: sum of |x|^p for p = 3 to 8, each power as a
-// product in fp64 (its first factor, the square of an fp32 value, is exact, so
-// p - 2 roundings, and none more than pow's at p = 3); kNormPow: sum of |x|^p in
-// fp64 through pow (any other p > 0), whose math the pass waits for: 1.0e8 bf16
-// elements 541 us through pow, as products 46 (p = 3), 58 (4) and 107 (8), p = 2
-// 30.
+// tensor.abs().max()); kNormInt + p - 3: sum of |x|^p for p = 3 to 8 (int_pow);
+// kNormPow: sum of |x|^p in fp64 through pow (any other p > 0), whose math the
+// pass waits for: 1.0e8 bf16 elements 541 us through pow, through int_pow 30 (p = 3
+// and 4, as p = 2), 47 (5), 48 (6), 52 (7) and 48 (8). A kind for each power: with
+// p an argument that every element branches on, 82 to 153 us.
 // x is the unscaled fp32 grad; every accumulation is in fp64.
 enum NormKind { kNormSq = 0, kNormAbs = 1, kNormMax = 2, kNormPow = 3, kNormInt = 4 };
 
@@ -369,17 +368,43 @@ __device__ __forceinline__ double norm_comb(double a, double b) {
   else return a + b;
 }
 
+// a^p for p = 3 to 8 and a >= 0 an fp32 value, to half an ulp: a^2 is exact in
+// fp64 and a^3 and a^4 are exact as the sum of a product and its rounding
+// error, so what is left is one product of such sums, whose own error joins the
+// small part before they are added. (A chain of p - 2 rounded products, the form
+// before, was up to 2 ulps off at p = 8.) An infinite a makes the small part NaN,
+// which fmin drops.
+template <int P>
+__device__ __forceinline__ double int_pow(double a) {
+  const double a2 = a * a;
+  double r, e;
+  if constexpr (P == 3) return a2 * a;
+  const double a3 = a2 * a, a3e = __builtin_fma(a2, a, -a3);
+  const double a4 = a2 * a2, a4e = __builtin_fma(a2, a2, -a4);
+  if constexpr (P == 4) return a4;
+  if constexpr (P == 5) {
+    r = a4 * a;
+    e = __builtin_fma(a4e, a, __builtin_fma(a4, a, -r));
+  } else if constexpr (P == 6) {
+    r = a3 * a3;
+    e = __builtin_fma(a3 + a3, a3e, __builtin_fma(a3, a3, -r));
+  } else if constexpr (P == 7) {
+    r = a4 * a3;
+    e = __builtin_fma(a4, a3e, __builtin_fma(a4e, a3, __builtin_fma(a4, a3, -r)));
+  } else {
+    r = a4 * a4;
+    e = __builtin_fma(a4 + a4, a4e, __builtin_fma(a4, a4, -r));
+  }
+  return r + fmin(e, __DBL_MAX__);
+}
+
 template <int K>
 __device__ __forceinline__ double norm_acc(double acc, float x, double p) {
   if constexpr (K == kNormSq) return __builtin_fma((double)x, (double)x, acc);
   else if constexpr (K == kNormAbs) return acc + fabs((double)x);
   else if constexpr (K == kNormMax) return norm_comb<K>(acc, fabs((double)x));
-  else if constexpr (K == kNormInt) {
-    const double a = fabs((double)x);
-    double r = a * a;
-    for (int k = 2; k < (int)p; ++k) r *= a;
-    return acc + r;
-  } else return acc + pow(fabs((double)x), p);
+  else if constexpr (K >= kNormInt) return acc + int_pow<K - kNormInt + 3>(fabs((double)x));
+  else return acc + pow(fabs((double)x), p);
 }
 
 // The elements of one 16-byte slot (8 16-bit grads or 4 fp32 grads).
@@ -581,7 +606,7 @@ __global__ __launch_bounds__(kBlock) void k_clip_prepare(const double* __restric
   if (threadIdx.x != 0) return;
   double norm = total;
   if constexpr (K == kNormSq) norm = sqrt(total);
-  else if constexpr (K == kNormPow || K == kNormInt) norm = pow(total, 1.0 / p);
+  else if constexpr (K == kNormPow) norm = pow(total, 1.0 / p);
   float coef = 1.0f;
   if (norm > max_norm) coef = (float)(max_norm / (norm + clip_eps));
   if (norm_out != nullptr) *norm_out = norm;
@@ -1974,7 +1999,7 @@ int norm_kind(double p, int* kind) {
   *kind = __builtin_isinf(p) ? kNormMax
           : p == 2.0         ? kNormSq
           : p == 1.0         ? kNormAbs
-          : p >= 3.0 && p <= 8.0 && p == floor(p) ? kNormInt
+          : p >= 3.0 && p <= 8.0 && p == floor(p) ? kNormInt + (int)p - 3
                                                   : kNormPow;
   return DSX_OK;
 }
@@ -1996,7 +2021,12 @@ void launch_norm(int kind, bool multi, const void* g, int64_t n, const DsxTensor
     case kNormSq: launch_norm_k<GD, kNormSq>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
     case kNormAbs: launch_norm_k<GD, kNormAbs>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
     case kNormMax: launch_norm_k<GD, kNormMax>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
-    case kNormInt: launch_norm_k<GD, kNormInt>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
+    case kNormInt + 0: launch_norm_k<GD, kNormInt + 0>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
+    case kNormInt + 1: launch_norm_k<GD, kNormInt + 1>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
+    case kNormInt + 2: launch_norm_k<GD, kNormInt + 2>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
+    case kNormInt + 3: launch_norm_k<GD, kNormInt + 3>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
+    case kNormInt + 4: launch_norm_k<GD, kNormInt + 4>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
+    case kNormInt + 5: launch_norm_k<GD, kNormInt + 5>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
     default: launch_norm_k<GD, kNormPow>(multi, g, n, t, c, nc, st, p, partials, nparts, s); break;
   }
 }
@@ -2028,8 +2058,7 @@ int do_clip_prepare(int kind, const double* partials, int32_t nparts, double nor
     case kNormSq: DSX_PREPARE(kNormSq); break;
     case kNormAbs: DSX_PREPARE(kNormAbs); break;
     case kNormMax: DSX_PREPARE(kNormMax); break;
-    case kNormInt: DSX_PREPARE(kNormInt); break;
-    default: DSX_PREPARE(kNormPow); break;
+    default: DSX_PREPARE(kNormPow); break;  // the integer powers' root too
   }
 #undef DSX_PREPARE
   return launch_status("dsx_clip_prepare");
