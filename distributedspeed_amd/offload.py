@@ -55,6 +55,7 @@ def _hip_runtime() -> ctypes.CDLL:
 
 def _free_pinned(hip: ctypes.CDLL, ptr: int) -> None:
     hip.hipDeviceSynchronize()  # no kernel may still be reading or writing it
+    del ops.host_blocks[ptr]
     hip.hipHostFree(ptr)
 
 
@@ -79,6 +80,7 @@ def pinned_empty(n: int) -> torch.Tensor:
         raise MemoryError(f"hipHostMalloc of {4 * n / 2**30:.1f} GiB failed (status {rc}): the pinned host memory "
                           "this machine allows is exhausted")
     buf = (ctypes.c_float * n).from_address(ptr.value)
+    ops.host_blocks[ptr.value] = 4 * n
     weakref.finalize(buf, _free_pinned, hip, ptr.value)
     return torch.from_numpy(np.ctypeslib.as_array(buf))
 
@@ -114,11 +116,6 @@ class HostStateStreamer:
         self.ev_out = [torch.cuda.Event() for _ in range(self.nbuf)]
         self.ev_step = torch.cuda.Event()  # the last run(), whatever stream it was on
         self.last_bytes = 0  # host<->HBM bytes the last run() moved (both directions)
-        self._held = ()  # the state that the last in-place run() steps
-
-    def __del__(self):
-        if getattr(self, "_held", ()):
-            self.ev_step.synchronize()  # the state may go with this streamer
 
     @staticmethod
     def _in_place(host_state) -> bool:
@@ -148,11 +145,6 @@ class HostStateStreamer:
         compute = torch.cuda.current_stream(self.device)
         compute.wait_event(self.ev_step)
         if not copy_only and self._in_place(host_state):
-            # A kernel's use of pinned memory is not known to torch's pinned
-            # allocator as a copy's is, so the arrays are kept until it is over.
-            if self._held and any(x is not y for x, y in zip(self._held, host_state)):
-                self.ev_step.synchronize()
-            self._held = tuple(host_state)
             for a, b, scal in pieces:
                 ops.adamw_host_state(*(t[a:b] for t in host_state),
                                      param16[a:b] if param16 is not None else None, grad[a:b], scal)

@@ -231,10 +231,23 @@ def plan_adamw_flat(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: tor
                   gdt, ctypes.c_int64(n), _ptr(scalars), keep=(master, exp_avg, exp_avg_sq, param16, grad, scalars))
 
 
+# Pinned blocks whose owner waits for the kernels on them before it frees them
+# (offload.pinned_empty): address -> bytes.
+host_blocks: dict[int, int] = {}
+
+
+def _kept_for_kernels(t: torch.Tensor) -> bool:
+    at = t.data_ptr()
+    return any(ptr <= at < ptr + nbytes for ptr, nbytes in list(host_blocks.items()))
+
+
 def adamw_host_state(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: torch.Tensor,
                      param16: torch.Tensor | None, grad: torch.Tensor, scalars: torch.Tensor) -> None:
     """K2 with the fp32 state in pinned host memory, in place over the host
-    link; param16, grad and scalars on the GPU whose stream it runs on."""
+    link; param16, grad and scalars on the GPU whose stream it runs on. The
+    caller may drop the state at once: torch's pinned allocator knows of copies
+    from its blocks but not of a kernel's use of them, so a copy of one element
+    follows on the same stream."""
     dev = _device(grad)
     n = grad.numel()
     host = torch.device("cpu")
@@ -249,6 +262,9 @@ def adamw_host_state(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: to
     _need(scalars, "scalars", torch.uint8, SCALARS_BYTES, dev, 8)
     _lib.call("dsx_adamw_host_state", _ptr(master), _ptr(exp_avg), _ptr(exp_avg_sq), _ptr(param16), pdt, _ptr(grad),
               gdt, ctypes.c_int64(n), _ptr(scalars), _stream(dev))
+    for t in (master, exp_avg, exp_avg_sq):
+        if n and not _kept_for_kernels(t):
+            torch.empty(1, dtype=t.dtype, device=dev).copy_(t.detach()[:1], non_blocking=True)
 
 
 def traffic_probe_flat(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: torch.Tensor,

@@ -115,3 +115,79 @@ def test_pinned_state_off_k2s_alignment_is_staged(gpu):
     for name, h, t in zip(("master", "exp_avg", "exp_avg_sq"), host, (p, m, v)):
         assert _bits(h, t), name
     assert _bits(o16, p16)
+
+
+def _busy(gpu):
+    """Work for the current stream that outlasts a few host calls by far."""
+    import torch
+    a = torch.ones(8192, 8192, device=gpu)
+    for _ in range(60):
+        a = (a @ a) * 0.0
+    done = torch.cuda.Event()
+    done.record()
+    return done
+
+
+def test_states_in_turn_do_not_block_the_host(gpu):
+    """Two states in turn, and fresh views of one, through one streamer: run()
+    returns while earlier work on the stream is still going on."""
+    import torch
+    from distributedspeed_amd import ops
+    from distributedspeed_amd.offload import HostStateStreamer
+    n = 10_008
+    p, m, v, p16, g = _inputs(n, torch.bfloat16, torch.bfloat16, gpu, 11)
+    states = [[_pinned(t) for t in (p, m, v)] for _ in range(2)]
+    outs = [p16.clone() for _ in states]
+    st = HostStateStreamer(gpu, 4096)
+    sc = _scalars(gpu)
+    _say("states in turn")
+    st.run(tuple(states[0]), outs[0], g, [(0, n, sc)])
+    torch.cuda.synchronize()
+    done = _busy(gpu)
+    st.run(tuple(states[1]), outs[1], g, [(0, n, sc)])
+    st.run(tuple(t[:] for t in states[0]), outs[0], g, [(0, n, sc)])
+    st.run(tuple(states[1]), outs[1], g, [(0, n, sc)])
+    assert not done.query()
+    torch.cuda.synchronize()
+    for _ in range(2):
+        ops.adamw_flat(p, m, v, p16, g, sc)
+    torch.cuda.synchronize()
+    for host, o16 in zip(states, outs):
+        assert all(_bits(h, t) for h, t in zip(host, (p, m, v))) and _bits(o16, p16)
+
+
+@pytest.mark.parametrize("torchs", [True, False])
+def test_state_dropped_behind_a_step_outlives_it(gpu, torchs):
+    """The streamer keeps no state, and a caller may drop it while the step is
+    still to come: torch's pinned allocator does not hand out its memory before,
+    and pinned_empty's is freed only then."""
+    import torch
+    import weakref
+    from distributedspeed_amd import ops
+    from distributedspeed_amd.offload import HostStateStreamer
+    n = 1 << 16
+    p, m, v, p16, g = _inputs(n, torch.bfloat16, torch.bfloat16, gpu, 12)
+    o16 = p16.clone()
+    host = [t.cpu().pin_memory() if torchs else _pinned(t) for t in (p, m, v)]
+    gone, homes = [weakref.ref(t) for t in host], [t.data_ptr() for t in host]
+    st = HostStateStreamer(gpu, 4096)
+    sc = _scalars(gpu)
+    spare = torch.full((n,), 7.0).pin_memory()  # written over whatever a too early reuse would give
+    torch.cuda.synchronize()
+    _say(f"dropped state, torch's allocator: {torchs}")
+    done = _busy(gpu)
+    st.run(tuple(host), o16, g, [(0, n, sc)])
+    del host
+    assert all(r() is None for r in gone)
+    if torchs:
+        new = [torch.empty(n, pin_memory=True) for _ in homes]
+        for t in new:
+            t.copy_(spare)
+        assert not done.query()
+        assert not {t.data_ptr() for t in new} & set(homes)
+    else:
+        assert done.query() and not set(homes) & set(ops.host_blocks)
+    ops.adamw_flat(p, m, v, p16, g, sc)
+    torch.cuda.synchronize()
+    assert _bits(o16, p16)
+    assert not torchs or all(torch.equal(t, spare) for t in new)
