@@ -49,13 +49,20 @@ def _hip_runtime() -> ctypes.CDLL:
         _hip.hipHostMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t, ctypes.c_uint]
         _hip.hipHostFree.restype = ctypes.c_int
         _hip.hipHostFree.argtypes = [ctypes.c_void_p]
-        _hip.hipDeviceSynchronize.restype = ctypes.c_int
+        for name in ("hipGetDevice", "hipSetDevice", "hipDeviceSynchronize"):
+            getattr(_hip, name).restype = ctypes.c_int
     return _hip
 
 
 def _free_pinned(hip: ctypes.CDLL, ptr: int) -> None:
-    hip.hipDeviceSynchronize()  # no kernel may still be reading or writing it
-    del ops.host_blocks[ptr]
+    # No kernel may still be reading or writing it, on whichever device.
+    _, devices = ops.host_blocks.pop(ptr)
+    here = ctypes.c_int()
+    hip.hipGetDevice(ctypes.byref(here))
+    for d in sorted(devices | {here.value}):
+        hip.hipSetDevice(d)
+        hip.hipDeviceSynchronize()
+    hip.hipSetDevice(here.value)
     hip.hipHostFree(ptr)
 
 
@@ -80,7 +87,7 @@ def pinned_empty(n: int) -> torch.Tensor:
         raise MemoryError(f"hipHostMalloc of {4 * n / 2**30:.1f} GiB failed (status {rc}): the pinned host memory "
                           "this machine allows is exhausted")
     buf = (ctypes.c_float * n).from_address(ptr.value)
-    ops.host_blocks[ptr.value] = 4 * n
+    ops.host_blocks[ptr.value] = (4 * n, set())
     weakref.finalize(buf, _free_pinned, hip, ptr.value)
     return torch.from_numpy(np.ctypeslib.as_array(buf))
 

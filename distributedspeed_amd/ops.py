@@ -232,13 +232,18 @@ def plan_adamw_flat(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: tor
 
 
 # Pinned blocks whose owner waits for the kernels on them before it frees them
-# (offload.pinned_empty): address -> bytes.
-host_blocks: dict[int, int] = {}
+# (offload.pinned_empty): address -> (bytes, indices of the devices they ran on).
+host_blocks: dict[int, tuple[int, set[int]]] = {}
 
 
-def _kept_for_kernels(t: torch.Tensor) -> bool:
+def _kept_for_kernels(t: torch.Tensor, device: torch.device) -> bool:
+    """Whether t lies in one of host_blocks, which notes its use on `device`."""
     at = t.data_ptr()
-    return any(ptr <= at < ptr + nbytes for ptr, nbytes in list(host_blocks.items()))
+    for ptr, (nbytes, devices) in list(host_blocks.items()):
+        if ptr <= at < ptr + nbytes:
+            devices.add(device.index)
+            return True
+    return False
 
 
 def adamw_host_state(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: torch.Tensor,
@@ -263,7 +268,7 @@ def adamw_host_state(master: torch.Tensor, exp_avg: torch.Tensor, exp_avg_sq: to
     _lib.call("dsx_adamw_host_state", _ptr(master), _ptr(exp_avg), _ptr(exp_avg_sq), _ptr(param16), pdt, _ptr(grad),
               gdt, ctypes.c_int64(n), _ptr(scalars), _stream(dev))
     for t in (master, exp_avg, exp_avg_sq):
-        if n and not _kept_for_kernels(t):
+        if n and not _kept_for_kernels(t, dev):
             torch.empty(1, dtype=t.dtype, device=dev).copy_(t.detach()[:1], non_blocking=True)
 
 

@@ -443,3 +443,55 @@ def test_rocprof_step_chains_count_the_parts_after_a_folded_first_part(tmp_path)
     assert three["kernels_us"]["k0_finalize"] == 4.0
     rag = res["ragged, two launches (K0 folded into K3)"]
     assert rag["steps"] == 3 and rag["kernels_us"]["k3_adamw_fold"] == 9.0
+
+
+# ---- pinned host memory -------------------------------------------------------------
+
+def test_pinned_memory_is_freed_after_the_kernels_of_every_device_that_used_it(monkeypatch):
+    """pinned_empty's finalizer against a recording HIP runtime: it waits for
+    each device that was given the memory (or a view of it) and for the current
+    one, which it leaves current, and then frees."""
+    import ctypes
+
+    from distributedspeed_amd import offload, ops
+
+    class Hip:
+        def __init__(self):
+            self.device, self.log, self.blocks = 0, [], []
+
+        def hipHostMalloc(self, out, nbytes, flags):
+            self.blocks.append(ctypes.create_string_buffer(nbytes))
+            out._obj.value = ctypes.addressof(self.blocks[-1])
+            return 0
+
+        def hipGetDevice(self, out):
+            out._obj.value = self.device
+            return 0
+
+        def hipSetDevice(self, d):
+            self.device = d
+            return 0
+
+        def hipDeviceSynchronize(self):
+            self.log.append(("wait", self.device))
+            return 0
+
+        def hipHostFree(self, ptr):
+            self.log.append(("free", ptr))
+            return 0
+
+    hip = Hip()
+    monkeypatch.setattr(offload, "_hip_runtime", lambda: hip)
+    a, b = offload.pinned_empty(100), offload.pinned_empty(100)
+    at_a, at_b = a.data_ptr(), b.data_ptr()
+    assert ops._kept_for_kernels(a[99:], torch.device("cuda", 1))
+    assert ops._kept_for_kernels(a, torch.device("cuda", 3))
+    assert not ops._kept_for_kernels(torch.zeros(4), torch.device("cuda", 1))
+    view = a[3:]
+    del a
+    assert hip.log == []  # a view still uses it
+    del view
+    assert hip.log == [("wait", 0), ("wait", 1), ("wait", 3), ("free", at_a)] and hip.device == 0
+    del b
+    assert hip.log[4:] == [("wait", 0), ("free", at_b)]
+    assert at_a not in ops.host_blocks and at_b not in ops.host_blocks
