@@ -125,11 +125,12 @@ class HostStateStreamer:
         self.last_bytes = 0  # host<->HBM bytes the last run() moved (both directions)
 
     @staticmethod
-    def _in_place(host_state) -> bool:
+    def _in_place(host_state, pieces) -> bool:
         """Whether K2 can take the state where it is: pinned, fp32 and
-        contiguous with every array on a 16-byte boundary, as K2 reads it."""
-        return all(t.is_pinned() and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
-                   for t in host_state)
+        contiguous with every piece on a 16-byte boundary, as K2 reads it."""
+        return (all(t.is_pinned() and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in host_state)
+                and all(a % 4 == 0 for a, _, _ in pieces))
 
     @property
     def stage(self) -> list:
@@ -151,7 +152,7 @@ class HostStateStreamer:
         param16, grad and the scalars are then unused."""
         compute = torch.cuda.current_stream(self.device)
         compute.wait_event(self.ev_step)
-        if not copy_only and self._in_place(host_state):
+        if not copy_only and self._in_place(host_state, pieces):
             for a, b, scal in pieces:
                 ops.adamw_host_state(*(t[a:b] for t in host_state),
                                      param16[a:b] if param16 is not None else None, grad[a:b], scal)

@@ -191,3 +191,28 @@ def test_state_dropped_behind_a_step_outlives_it(gpu, torchs):
     torch.cuda.synchronize()
     assert _bits(o16, p16)
     assert not torchs or all(torch.equal(t, spare) for t in new)
+
+
+@pytest.mark.parametrize("start", [1, 2, 3, 4, 7])
+def test_a_piece_off_k2s_alignment_is_staged(gpu, start):
+    """A piece that starts where the 16-bit buffers are aligned and the fp32
+    state is not (4 elements in, both are): staged, as every piece once was."""
+    import torch
+    from distributedspeed_amd import ops
+    from distributedspeed_amd.offload import HostStateStreamer
+    n = 9_001
+    p, m, v, p16, g = _inputs(n, torch.bfloat16, torch.bfloat16, gpu, 13)
+    host = [_pinned(t) for t in (p, m, v)]
+    pad = 8 - start
+
+    def at(t):  # t's values with element `start` on a 16-byte boundary
+        return torch.cat([t[:1].expand(pad), t])[pad:]
+
+    o16, og = at(p16), at(g)
+    _say(f"piece from {start}")
+    HostStateStreamer(gpu, 4096).run(tuple(host), o16, og, [(start, n, _scalars(gpu))])
+    rest = [t[start:].clone() for t in (p, m, v, p16, g)]
+    ops.adamw_flat(*rest, _scalars(gpu))
+    torch.cuda.synchronize()
+    for h, t, new in zip(host + [o16], (p, m, v, p16), rest):
+        assert _bits(h[:start], t[:start]) and _bits(h[start:], new)
