@@ -1319,9 +1319,9 @@ __device__ __forceinline__ Sc scalars_rec(const DsxStepScalars* scalars, int32_t
 // current chunk's tensor record, so that it is in by the time the current
 // chunk is done.
 //
-// NP > 1: the grads are at the addresses in gp, by tensor, and the last block
-// also stores those in the table's records, for the launches after this one (a
-// small list whose grads moved: one launch less than k_set_grads and K1, the
+// NP > 1: the grads of the first `count` tensors are at the addresses in gp, and
+// the last block also stores those in the table's records, which no block of this
+// launch reads, for the launches after this one (a small list whose grads moved: one launch less than k_set_grads and K1, the
 // MLP's list 22.5 -> 18.3 us a step).
 template <int GD, bool WAVE, int NP>
 __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorRef* __restrict__ tensors,
@@ -1346,7 +1346,7 @@ __global__ __launch_bounds__(kBlock) void k1_unscale_norm_multi(const DsxTensorR
   if (c < nchunks) {  // the grid is the partial count, which may exceed the chunk count
     DsxChunk ch = chunk_rec(chunks, c);
     for (;;) {
-      const void* base = NP > 1 ? gp.g[ch.tensor] : tensor_rec(tensors, ch.tensor).grad;
+      const void* base = NP > 1 && ch.tensor < count ? gp.g[ch.tensor] : tensor_rec(tensors, ch.tensor).grad;
       const typename G::elem* g = static_cast<const typename G::elem*>(base) + ch.start;
       const int64_t cn = c + stride;
       const DsxChunk chn = chunk_rec(chunks, cn < nchunks ? cn : c);

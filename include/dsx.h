@@ -562,10 +562,11 @@ int dsx_zero_step_multi(const DsxTensorRef* tensors, const DsxChunk* chunks,
                         const DsxGroupsDev* groups /* host */, double* partials,
                         int32_t nparts, DsxStepScalars* out, void* stream);
 
-/* dsx_zero_step_multi for a list whose grads have moved to the addresses in
- * grads[ntensors] (a HOST array, read before the call returns; at most 64
- * tensors, which is all of the list): as dsx_set_grads and then the step, with
- * the addresses carried by the step's first launch. */
+/* dsx_zero_step_multi for a list the grads of whose first ntensors tensors (1
+ * to 64, and no more than the table holds) have moved to the addresses in
+ * grads[ntensors] (a HOST array, read before the call returns): as
+ * dsx_set_grads and then the step, with the addresses carried by the step's
+ * first launch. */
 int dsx_zero_step_multi_moved(DsxTensorRef* tensors, const DsxChunk* chunks,
                               int64_t nchunks, int64_t numel, int param_dtype,
                               int grad_dtype, DsxState* state,

@@ -244,3 +244,46 @@ def test_moving_grads_reach_every_launch(gpu, k, size):
         assert _bits(pf.data, pr.data)
         for key in ("master", "exp_avg", "exp_avg_sq"):
             assert _bits(opts[0][1].state[pf][key], opts[1][1].state[pr][key]), key
+
+
+@pytest.mark.parametrize("count", [1, 3, 5])
+def test_moved_grads_of_the_first_tensors(gpu, count):
+    """dsx_zero_step_multi_moved with the new addresses of the list's first
+    tensors: the others' grads stay where the table has them."""
+    import ctypes
+    import torch
+    from distributedspeed_amd import _lib, ops
+    from distributedspeed_amd.optimizers import MultiTensorAdamWOptimizer
+    _say(f"moved grads of the first {count} of 5")
+    sizes = (5000, 3, 8193, 70_001, 16)
+    gen = torch.Generator(device=gpu).manual_seed(4)
+    init = [torch.empty(k, device=gpu).normal_(0.0, 0.02, generator=gen) for k in sizes]
+    grads = [[torch.empty(k, device=gpu).normal_(0.0, 1e-3, generator=gen).half() for k in sizes] for _ in range(2)]
+    taken = grads[1][:count] + grads[0][count:]
+
+    def make(gs):
+        ps = [torch.nn.Parameter(t.clone()) for t in init]
+        opt = MultiTensorAdamWOptimizer(ps, lr=1e-3, param_dtype=torch.float16, device=gpu, max_grad_norm=1.0)
+        for p, g in zip(ps, gs):
+            p.grad = g
+        return ps, opt
+
+    (pa, a), (pb, b) = make(grads[0]), make(taken)
+    b.step()
+    a._plans()  # the table over grads[0]
+    a.steps_issued += 1
+    a._refresh_group_block()
+    table = a.store.table()
+    assert table.nchunks > 0 and a.store.small_table is None
+    _lib.call("dsx_zero_step_multi_moved", table.tensors.data_ptr(), table.chunks.data_ptr(), table.nchunks, table.numel,
+              table.pdt, table.gdt, a.dstate.data_ptr(), a.scaler.to_c(), ctypes.byref(a._gblock),
+              a.partials.data_ptr(), a.nparts, a.scalars.data_ptr(),
+              (ctypes.c_void_p * count)(*[g.data_ptr() for g in grads[1][:count]]), count, ops.stream_of(gpu))
+    torch.cuda.synchronize()
+    assert bytes(a.read_state()) == bytes(b.read_state())
+    for x, y in zip(pa, pb):
+        assert _bits(x.data, y.data)
+        for key in ("master", "exp_avg", "exp_avg_sq"):
+            assert _bits(a.state[x][key], b.state[y][key]), key
+    refs = (_lib.DsxTensorRef * len(sizes)).from_buffer_copy(bytes(table.tensors.cpu().numpy()))
+    assert [r.grad for r in refs] == [g.data_ptr() for g in taken]
