@@ -448,14 +448,14 @@ __device__ __forceinline__ float inv_of(float scale) {
 // Every grad is read twice in a step: by the norm pass, then by the update.
 // A load with the nontemporal hint passes the 256 MB memory-side cache by, a
 // plain one leaves its line there, and the update's own streams (all
-// nontemporal) do not evict it. So the norm passes read the first
-// kKeepBytes of the grads, in the order in which the update takes them, with
-// plain loads and the rest, which would only evict those, nontemporally; the
-// update's grad loads then find them in the cache: 2 of the step's 30 bytes an
-// element (4 of 32 with fp32 grads) do not come from HBM again. Flat steps on
-// MI355X, one process, with 0 / 128 / 192 / 256 / 320 MB kept and with every
-// load plain, us: 1.24e8 bf16 elements (248 MB of grads) 616 / 599 / 591 /
-// 584 / 584 / 584; 6.0e7 fp32 (240 MB) 320 / 307 / 298 / 293 / 293 / 293;
+// nontemporal) do not evict it. So the norm passes read the first kKeepBytes of
+// the grads (of a list, in the order of its chunks, whatever part of it the update
+// begins with) with plain loads and the rest, which would only evict those,
+// nontemporally; the update's grad loads then find them in the cache: 2 of the
+// step's 30 bytes an element (4 of 32 with fp32 grads) do not come from HBM again.
+// Flat steps on MI355X, one process, with 0 / 128 / 192 / 256 / 320 MB kept and
+// with every load plain, us: 1.24e8 bf16 elements (248 MB of grads) 616 / 599 /
+// 591 / 584 / 584 / 584; 6.0e7 fp32 (240 MB) 320 / 307 / 298 / 293 / 293 / 293;
 // 2.5e8 bf16 (500 MB) 1246 / 1228 / 1219 / 1209 / 1209 / 1210; 1.0e9 bf16
 // 4981 / 4958 / 4951 / 4940 / 4940 / 4971. Below 3e6 elements both are the same.
 constexpr int64_t kKeepBytes = int64_t(1) << 28;
@@ -675,9 +675,11 @@ __global__ __launch_bounds__(kBlock) void k1_copy_unscale_norm(const void* __res
 // out[b] = sum of partials[offsets[b] .. offsets[b + 1]), by block b, each
 // thread over a fixed stride and the block reduce in a fixed tree: the same
 // bits for the same partials.
-// fold != NULL: block 0 starts a folded step, as k1_unscale_norm does (a training
-// iteration of the 784-1024-1024-10 MLP 432 -> 410 us, K0 a launch of its own and
-// three calls from Python against one).
+// fold != NULL: block 0 starts a folded step, as k1_unscale_norm does, so that K0
+// needs no launch of its own and the step is one call from Python instead of three
+// (a training iteration of 4 blocks 512 -> 2048 -> 512, alternated in one process, 733 ->
+// 717 us; of the 784-1024-1024-10 MLP, which the host bounds, 432 -> 410 there, but
+// in processes of its own runs of one side differ by 13-25%, which shows nothing).
 __global__ __launch_bounds__(kBlock) void k_reduce_segments(const double* __restrict__ partials,
                                                             const int64_t* __restrict__ offsets,
                                                             double* __restrict__ out, DsxState* fold) {
@@ -1093,15 +1095,26 @@ __device__ __forceinline__ const DsxGroupsDev& group_block(const DsxGroupsDev* g
 // 79.2; from 9e7 on slower, 428 -> 436). kFoldKeep, while the fp32 state is at
 // most kKeepStateBytes: the stores are also written through to the
 // memory-side cache (scope bit sc1) instead of past it, so that the next step's
-// loads find the state there if what ran in between has not displaced it, and
-// no dirty lines are left in the L2s for the kernel's end to write back (plain
-// stores: 14.4 against 12.6 us at 1.9e6 elements). us with three states in turn
-// / one state again and again, kFoldSmall against kFoldKeep: 1.9e6 elements
-// 13.9 / 11.2 against 12.6 / 12.0, 2.5e6 18.0 / 15.3 against 15.6 / 14.8, 4.0e6
-// 25.1 / 23.7 against 22.4 / 21.6, 5.0e6 30.1 / 28.5 against 27.1 / 26.0; from
-// 7.1e6 on only one state alone gains (39.3 / 38.7 against 40.1 / 34.9, 1.6e7
-// 79.2 / 78.6 against 82.0 / 72.9), which a training step in between would
-// displace. kFoldPlain: the nontemporal hint switched off.
+// loads, and the forward's of the 16-bit parameters, find what it wrote there
+// unless what ran in between has displaced it, and no dirty lines are left in the
+// L2s for the kernel's end to write back (plain stores: 14.4 against 12.6 us at
+// 1.9e6 elements). What runs between steps decides what that gives. Flat bf16
+// steps, kFoldSmall / kFoldKeep, alternated in one process, us an iteration less
+// the same iteration without its step:
+//   elements                          9.0e5        1.9e6        4.2e6        5.5e6
+//   forward, backward of 64 rows   19.4 / 15.3  25.4 / 17.5  50.3 / 35.5  47.1 / 36.4
+//   the same of 2048 rows          14.4 / 12.0  24.8 / 15.2  36.0 / 23.5  51.6 / 29.7
+//   of 16384 rows                  15.7 / 12.4  17.9 / 14.7  31.1 / 30.9  40.2 / 28.2
+//   nothing, one state              9.5 /  9.4  11.4 / 11.9  23.6 / 22.3  30.3 / 28.6
+//   nothing, three states in turn   9.3 /  9.5  12.8 / 12.6  25.5 / 23.0  31.8 / 30.8
+//   512 MB read and written        11.2 / 15.1  14.8 / 19.0  28.9 / 31.5  36.2 / 40.1
+// (the model: square layers, three of 9.0e5 and 1.9e6 elements, four of the
+// others; lists and 3.0e5 elements alike). It gains in a training iteration, and
+// costs 2.5-5 us where a pass over twice the cache displaces the state: the line
+// is drawn for the former. It lies at 5.6e6 elements because above, several states
+// in turn no longer gain (a list of 7.1e6 39.6 / 41.1, of 1.6e7 80.0 / 85.3; one
+// model's iterations still do there: 7.1e6 after 2048 rows 49.4 / 35.5, 1.6e7
+// 108 / 86). kFoldPlain: the nontemporal hint switched off.
 enum FoldPolicy { kFoldPlain = 0, kFoldStream = 1, kFoldSmall = 2, kFoldKeep = 3 };
 constexpr int64_t kKeepStateBytes = int64_t(1) << 26;
 
@@ -2358,7 +2371,10 @@ int do_k3_fold(const List& l, int64_t step_elems, int pdt, int gdt, const double
 // K3's first chunks, about kFoldFirstElems elements, or the first K2 tensor's
 // first part (us a step against K0 as a launch of its own and the rest called
 // from Python one by one: 4.0e7 bf16 elements 222 -> 204, 8.0e7 414 -> 395, 1.5e8
-// 763 -> 735, 2.5e8 1275 -> 1233). Else K0 is a launch of its own.
+// 763 -> 735, 2.5e8 1275 -> 1233). Else K0 is a launch of its own: with more
+// partials than a block reduces, in tables of smaller chunks than the rule's, and
+// in lists within the fold's bound that have a K2 tensor (2.1e7 to 2.5e7 elements
+// with a tensor of at least 2^24), where folding it was not measured.
 int list_step(const List& norm, const List& k3, const DsxTensorRef* k2, int32_t nk2, int64_t numel, int pdt, int gdt,
               DsxState* state, const DsxScalerConfig& scaler, const DsxGroupsDev* groups, double* partials,
               int32_t nparts, DsxStepScalars* out, hipStream_t s, const MovedGrads* moved = nullptr) {
