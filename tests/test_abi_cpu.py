@@ -277,6 +277,145 @@ def test_argument_checks_reject_before_launch(lib):
     assert lib.dsx_set_tuning_multi(0, 1, 1, 2) == EINVAL
 
 
+def test_one_call_forms_reject_before_launch(lib):
+    """The one-call clip, the step over split lists, with moved grads and from
+    the hand-over's segments, the grad addresses and the step on host state:
+    DSX_EINVAL for every bad argument, before any HIP call."""
+    from distributedspeed_amd import _lib
+    EINVAL = _lib.DSX_EINVAL
+    al = 1 << 20
+
+    def refused(rc, text):
+        assert rc == EINVAL and text in lib.dsx_last_error(), (rc, lib.dsx_last_error())
+
+    # clip_grad_norm_ in one call, both forms
+    def clip(grad=al, gdt=2, n=16, p=2.0, max_norm=1.0, eps=1e-6, partials=al, nparts=1, state=al, out=al):
+        return lib.dsx_clip_grad_norm(grad, gdt, n, p, max_norm, eps, partials, nparts, state, out, None)
+
+    def clip_multi(tensors=al, chunks=al, nchunks=1, gdt=2, p=2.0, max_norm=1.0, eps=1e-6, partials=al, nparts=1,
+                   state=al, out=al):
+        return lib.dsx_clip_grad_norm_multi(tensors, chunks, nchunks, gdt, p, max_norm, eps, partials, nparts, state,
+                                            out, None)
+
+    for f in (clip, clip_multi):
+        for bad in (0.0, -2.0, float("nan")):
+            refused(f(p=bad), b"norm_type")
+        refused(f(max_norm=-1.0), b"max_norm")
+        refused(f(max_norm=float("nan")), b"max_norm")
+        refused(f(eps=-1.0), b"clip_eps")
+        refused(f(state=None), b"state")
+        refused(f(out=None), b"norm_out")
+        refused(f(gdt=7), b"dtype")
+        refused(f(nparts=0), b"")
+        refused(f(nparts=_lib.DSX_MAX_PARTIALS + 1), b"")
+        refused(f(partials=None), b"")
+    refused(clip(n=-1), b"n must be")
+    refused(clip(grad=al + 2), b"aligned")
+    refused(clip_multi(nchunks=-1), b"chunk table")
+    refused(clip_multi(chunks=None), b"chunk table")
+
+    # the grads' addresses
+    ptrs = (ctypes.c_void_p * 65)(*([al] * 65))
+    refused(lib.dsx_set_grads(al, ptrs, -1, None), b"grads")
+    refused(lib.dsx_set_grads(None, ptrs, 1, None), b"grads")
+    refused(lib.dsx_set_grads(al, None, 1, None), b"grads")
+
+    # the list steps
+    scfg = _lib.DsxScalerConfig(0, 1000, 1, 0, 1.0, 2.0, 0.5, 0.0)
+    gb = _lib.DsxGroupsDev()
+    gb.ngroups, gb.bc_len = 2, 4
+    for k in range(2):
+        gb.hyper[k] = _lib.DsxAdamwHyper(1e-3, 0.9, 0.999, 1e-8, 0.0, 0.0, 1e-6)
+        gb.bc_table[k] = al
+    g = ctypes.byref(gb)
+
+    def moved(tensors=al, chunks=al, nchunks=1, numel=16, pdt=1, gdt=1, state=al, groups=g, partials=al, nparts=1,
+              out=al, grads=ptrs, count=1):
+        return lib.dsx_zero_step_multi_moved(tensors, chunks, nchunks, numel, pdt, gdt, state, scfg, groups, partials,
+                                             nparts, out, grads, count, None)
+
+    k2 = (_lib.DsxTensorRef * 2)()
+    for r in k2:
+        r.master = r.exp_avg = r.exp_avg_sq = r.param16 = r.grad = al
+        r.numel = 64
+
+    def lists(tensors=al, chunks=al, nchunks=1, numel=144, k3=(al, al, 1, 16), refs=k2, nk2=2, pdt=1, gdt=1, state=al,
+              groups=g, partials=al, nparts=1, out=al):
+        return lib.dsx_zero_step_lists(tensors, chunks, nchunks, numel, *k3, refs, nk2, pdt, gdt, state, scfg, groups,
+                                       partials, nparts, out, None)
+
+    for count in (-1, 0, 65):
+        refused(moved(count=count), b"ntensors")
+    refused(moved(grads=None), b"grads")
+    refused(moved(tensors=None), b"grads")
+    for f in (moved, lists):
+        refused(f(gdt=7), b"grad dtype")
+        refused(f(pdt=0), b"param16 dtype")
+        refused(f(nchunks=-1), b"chunk table")
+        refused(f(chunks=None), b"chunk table")
+        refused(f(numel=-1), b"numel")
+        refused(f(state=None), b"null state")
+        refused(f(groups=None), b"null state")
+        refused(f(out=None), b"null state")
+        refused(f(nparts=0), b"")
+        refused(f(partials=None), b"")
+    refused(lists(k3=(None, al, 1, 16)), b"chunk table")
+    refused(lists(k3=(al, al, -1, 16)), b"chunk table")
+    refused(lists(k3=(al, al, 1, -16)), b"numel")
+    refused(lists(nk2=-1), b"K2 tensors")
+    refused(lists(refs=None), b"K2 tensors")
+    for field, bad, text in (("group", -1, b"group"), ("group", 2, b"group"), ("master", al + 4, b"aligned"),
+                             ("exp_avg", al + 8, b"aligned"), ("exp_avg_sq", al + 4, b"aligned"),
+                             ("param16", al + 2, b"aligned"), ("grad", al + 2, b"aligned"), ("grad", None, b"null"),
+                             ("numel", -1, b"n must be")):
+        good = getattr(k2[1], field)
+        setattr(k2[1], field, bad)
+        refused(lists(), text)
+        setattr(k2[1], field, good)
+    gb.hyper[1].eps = -1.0
+    refused(moved(), b"epsilon")
+    refused(lists(), b"epsilon")
+    gb.hyper[1].eps = 1e-8
+    gb.ngroups = 0
+    refused(lists(), b"ngroups")
+    gb.ngroups = 2
+
+    # the step from the hand-over's segments
+    plan = _lib.DsxFlatPlan(al, al, al, al, al, 64, 2, 2, al, al, al, 4, 2)
+    plan.scaler = scfg
+    plan.group_end[0], plan.group_end[1] = 32, 64
+
+    def segments(p=ctypes.byref(plan), groups=g, block=al, offsets=al, partials=al, nseg=4):
+        return lib.dsx_zero_step_segments(p, groups, block, offsets, partials, nseg, None)
+
+    refused(segments(p=None), b"null plan")
+    refused(segments(groups=None), b"null plan")
+    refused(segments(block=None), b"block partials")
+    refused(segments(offsets=None), b"offsets")
+    refused(segments(partials=None), b"")
+    refused(segments(nseg=0), b"")
+    refused(segments(nseg=_lib.DSX_MAX_PARTIALS + 1), b"")
+    plan.group_end[0] = 36
+    refused(segments(), b"group_end")
+    plan.group_end[0] = 32
+    gb.ngroups = 1
+    refused(segments(), b"groups")
+    gb.ngroups = 2
+
+    # the step on host state: what the flat update refuses, before the memory is looked at
+    def host(master=al, grad=al, gdt=2, n=16, p16=al, scalars=al):
+        return lib.dsx_adamw_host_state(master, al, al, p16, 2, grad, gdt, n, scalars, None)
+
+    refused(host(n=-1), b"n must be")
+    refused(host(master=al + 4), b"aligned")
+    refused(host(grad=al + 2), b"aligned")
+    refused(host(p16=al + 2), b"aligned")
+    refused(host(grad=None), b"null")
+    refused(host(gdt=7), b"grad dtype")
+    refused(host(scalars=None), b"null scalars")
+    assert host(n=0) == 0
+
+
 def test_python_layer_mirrors_torch_errors():
     from distributedspeed_amd.flat_step import AdamWHyper, ScalerConfig
     with pytest.raises(ValueError, match="Invalid learning rate"):

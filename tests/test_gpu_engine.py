@@ -418,10 +418,10 @@ def test_initialize_refuses_multi_rank(gpu, monkeypatch):
 
 def test_offloaded_state_matches_in_hbm_step(gpu):
     """configs[4]'s path at reduced size: master/m/v in pinned host memory,
-    streamed through HBM in small chunks (so that every stage of the copy-in /
-    K2 / copy-out pipeline wraps around its buffers several times), two
-    parameter groups, fp16 dynamic scaling with an overflow step. Results are
-    bit-identical to the same steps with the state in HBM."""
+    stepped there in place (the staging of other host memory:
+    test_gpu_offload_in_place.py), two parameter groups, fp16 dynamic scaling
+    with an overflow step. Results are bit-identical to the same steps with the
+    state in HBM."""
     import torch
     from distributedspeed_amd.flat_step import ScalerConfig
     from distributedspeed_amd.optimizers import AdamWOptimizer

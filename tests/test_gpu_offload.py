@@ -1,20 +1,19 @@
 """the Llama-3-70B ZeRO-3 one-rank shard whose fp32
-master / exp_avg / exp_avg_sq live in pinned host memory and stream through
-HBM in 64 Mi-element chunks (the optimizer's default offload_chunk_elems),
-with bf16 grads N(0, 3e-4^2) and bf16 params in HBM, AdamW lr 1.5e-4, betas
-(0.9, 0.95), eps 1e-8, weight decay 0.1, clipping at 1.0.
+master / exp_avg / exp_avg_sq live in pinned host memory, where the step
+reads and writes them in place, with bf16 grads N(0, 3e-4^2) and bf16 params
+in HBM, AdamW lr 1.5e-4, betas (0.9, 0.95), eps 1e-8, weight decay 0.1,
+clipping at 1.0.
 
 The full shard (8.82e9 elements, 105.8 GB of state) exceeds what this
 machine pins (no single hipHostMalloc above 32 GiB, about 64 GiB in all), so
 the test runs the benchmark's shard, the largest its 32 GiB pinned budget
 holds (42 chunks' worth): 2,818,564,633 parameters (2,818,564,640 elements
 with the 8-element alignment) in two parameter groups (the second with lr
-3e-4 and no weight decay), each ending in a ragged partial chunk, 43 chunks
-in all, so the three staging buffers wrap around fourteen times. Three
-steps, the second with an inf grad (skipped: bf16 has no loss scale, but a non-finite
-grad still skips). After the first and the last step the offloaded state and
-params are compared bit for bit with the oracle (ZeroStepOracle with both
-groups) and with the same steps run with the state in HBM
+3e-4 and no weight decay), neither a multiple of 64 Mi elements. Three
+steps, the second with an inf grad (skipped: bf16 has no loss scale, but a
+non-finite grad still skips). After the first and the last step the offloaded
+state and params are compared bit for bit with the oracle (ZeroStepOracle with
+both groups) and with the same steps run with the state in HBM
 (Src/zero/stage1.py:376-398, 482-498 and Src/zero/stage3.py:881-898,
 1189-1207 are the reference's offload patterns)."""
 from __future__ import annotations

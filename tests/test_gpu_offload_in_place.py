@@ -1,7 +1,7 @@
 """K2 on fp32 state in pinned host memory (dsx_adamw_host_state): the same bits
 as K2 on the same state in HBM, at the edges of its slots, trips and grid, and
 through the offloaded step; host memory that is not pinned is refused by the
-entry point and staged by the streamer."""
+entry point and staged by the streamer, as is pinned memory off K2's alignment."""
 from __future__ import annotations
 
 import sys
@@ -98,19 +98,27 @@ def test_the_streamer_takes_pinned_and_pageable_state(gpu, pinned):
     assert _bits(o16, p16)
 
 
-def test_pinned_state_off_k2s_alignment_is_staged(gpu):
+@pytest.mark.parametrize("n,cut,nbuf", [(9_001, 0, 3), (10 * 4096 + 41, 5 * 4096 + 24, 3),
+                                        (10 * 4096 + 41, 5 * 4096 + 24, 2)])
+def test_pinned_state_off_k2s_alignment_is_staged(gpu, n, cut, nbuf):
     """Views that start 4 bytes into a pinned array: K2 reads 16 bytes at a
-    time, so they take the staged path, as all pinned state once did."""
+    time, so they take the staged path, as all pinned state once did. The larger
+    ones are two pieces of 6 chunks each, two steps on end: every staging slot is
+    filled, stepped and emptied four times a step or more, with copies that the
+    host does not wait for."""
     import torch
     from distributedspeed_amd.offload import HostStateStreamer
-    n = 9_001
     p, m, v, p16, g = _inputs(n, torch.bfloat16, torch.bfloat16, gpu, 5)
     host = [_pinned(torch.cat([t[:1], t]))[1:] for t in (p, m, v)]
     o16 = p16.clone()
-    st = HostStateStreamer(gpu, 4096)
-    st.run(tuple(host), o16, g, [(0, n, _scalars(gpu))])
+    st = HostStateStreamer(gpu, 4096, nbuf)
+    pieces = [(a, b, _scalars(gpu)) for a, b in ((0, cut), (cut, n)) if b > a]
+    for _ in range(2):
+        st.run(tuple(host), o16, g, pieces)
+    assert st._stage is not None and st.last_bytes == 24 * n
     from distributedspeed_amd import ops
-    ops.adamw_flat(p, m, v, p16, g, _scalars(gpu))
+    for _ in range(2):
+        ops.adamw_flat(p, m, v, p16, g, _scalars(gpu))
     torch.cuda.synchronize()
     for name, h, t in zip(("master", "exp_avg", "exp_avg_sq"), host, (p, m, v)):
         assert _bits(h, t), name
