@@ -385,8 +385,8 @@ def measure_dropin_headline(dev, n: int, steps: int, warmup: int, headline_ms: f
             "storage": "f32 state / bf16 grads+params", "numel": n, "steps": steps, "warmup": warmup,
             "path": "dsx_zero_step_plan: " + ("K1, then K2 with K0's finalize folded into every block"
                                                if n <= 3 << 23 else
-                                               f"K1, then K2 in {k2_parts(n, None)} parts with K0's finalize "
-                                               "folded into the first"),
+                                               "K1, then K2 with K0's finalize folded into the first 2^24 elements "
+                                               f"and the rest in {k2_parts(n - (1 << 24), None)} parts"),
             "headline_ms_per_step": round(headline_ms, 4) if headline_ms else None, "modes": out}
 
 

@@ -14,8 +14,8 @@ built once and the copies disappear:
 
 With fp32 training there is no param16: param.data are views of master and
 grads are fp32. With `offload=True` master / exp_avg / exp_avg_sq are pinned
-host tensors instead (the step streams them through HBM; param16 and grad
-stay in HBM), which needs a 16-bit param dtype.
+host tensors instead (the step reads and writes them there over the host link;
+param16 and grad stay in HBM), which needs a 16-bit param dtype.
 
 Grads reach the flat buffer one of two ways. After zero_grad(set_to_none=
 False) the views stay bound and autograd accumulates into them: a zeroing

@@ -39,8 +39,8 @@ class GraphedStep:
 
     def __init__(self, opt):
         if opt.streamer is not None:
-            raise NotImplementedError("graph capture covers HBM-resident state; the offloaded step streams "
-                                      "host chunks under host control")
+            raise NotImplementedError("graph capture covers HBM-resident state; the offloaded step's is in host "
+                                      "memory")
         dev = opt.device
         self.device = dev
         self.ngroups = len(opt.param_groups)

@@ -122,7 +122,9 @@ class HostStateStreamer:
         self.ev_done = [torch.cuda.Event() for _ in range(self.nbuf)]
         self.ev_out = [torch.cuda.Event() for _ in range(self.nbuf)]
         self.ev_step = torch.cuda.Event()  # the last run(), whatever stream it was on
-        self.last_bytes = 0  # host<->HBM bytes the last run() moved (both directions)
+        # host<->HBM bytes of the last run() (both directions); in place, of a step
+        # that was not skipped: a skipped one moves none
+        self.last_bytes = 0
 
     @staticmethod
     def _in_place(host_state, pieces) -> bool:

@@ -370,8 +370,8 @@ class _FusedAdamWBase(torch.optim.Optimizer):
         exp_avg / exp_avg_sq / step) plus the fp32 master and the device
         scaler state; tensors are host copies."""
         if getattr(self, "streamer", None) is not None:
-            # offloaded state: pinned host memory written by asynchronous
-            # copies, whichever stream the caller is on now
+            # offloaded state: pinned host memory that the step's kernels write,
+            # whichever stream the caller is on now
             torch.cuda.synchronize(self.device)
         s = self.read_state()
         groups = []
@@ -453,7 +453,10 @@ class _FusedAdamWBase(torch.optim.Optimizer):
 
 class AdamWOptimizer(_FusedAdamWBase):
     """The flat form: every parameter re-homed into one FlatPartition (the
-    reference's contiguous_gradients layout, Src/zero/stage2.py:108-193)."""
+    reference's contiguous_gradients layout, Src/zero/stage2.py:108-193).
+    offload_chunk_elems: the chunk of self.streamer's staged path, which only
+    state that is not pinned takes; the partition's own is pinned and stepped in
+    place, so it changes nothing in a step."""
 
     def __init__(self, params: Iterable, lr: float = 1e-3, betas=(0.9, 0.999), eps: float = 1e-8,
                  weight_decay: float = 1e-2, *, max_grad_norm: float = 0.0, param_dtype: torch.dtype | None = None,
@@ -650,9 +653,9 @@ class AdamWOptimizer(_FusedAdamWBase):
         self.flat.disarm_hook_norm()
         self._after_finalize()
         if self.streamer is not None:
-            # State in pinned host memory: stream it through HBM chunk by chunk.
-            # A skipped step streams too (K2 leaves the chunks unchanged), which
-            # keeps the host free of any wait on the device.
+            # State in pinned host memory: K2 reads and writes it there over the
+            # host link; on a skipped step it returns at once, so that nothing
+            # moves and the host waits for nothing.
             pieces = [(a, b, self.scalars[gi * ops.SCALARS_BYTES:(gi + 1) * ops.SCALARS_BYTES])
                       for gi, (a, b) in enumerate(self.flat.group_ranges) if b > a]
             self.streamer.run((self.flat.master, self.flat.exp_avg, self.flat.exp_avg_sq), self.flat.param16,
